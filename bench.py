@@ -166,17 +166,14 @@ def lu_roofline(ms, nsys, N, KL, KU, kernel="k_gbtrf<double>", rhs=False):
 
 def lu_kernel_name(KL, KU, fused_ut=False):
     """The factorization kernel the library dispatches for this band shape
-    (the one-wave register kernel for the channel shapes unless
+    (the one-wave panel kernel for the channel shapes unless
     SZ_GBTRF_KERNEL selects the LDS window kernel); fused_ut: the variant
     that also solves U^T y = b (a fresh factorization followed by one
     transposed solve, as in every implicit substep)."""
     sel = os.environ.get("SZ_GBTRF_KERNEL", "")
     if sel.startswith("l") or (KL, KU) not in ((34, 34), (24, 24), (34, 20)):
         return "k_gbtrf<double, 256>"
-    if fused_ut:
-        return f"k_gbtrf_wave<double, {KL + 1}, {KL + KU}, 4, true>"
-    bs = {"v2": 2, "v4": 4}.get(sel, 8)
-    return f"k_gbtrf_wave<double, {KL + 1}, {KL + KU}, {bs}>"
+    return f"k_gbtrf_panel<double, {KL + 1}, {KL + KU}, {str(fused_ut).lower()}>"
 
 
 # HBM bytes per LU launch measured with FETCH_SIZE/WRITE_SIZE PMC passes and
@@ -764,7 +761,7 @@ def main_rk3(args):
     out["config1_solve"] = solve_workload(max(10, args.steps // 2), 3,
                                           cpu=not args.no_cpu)
     if not args.no_traffic:
-        t, why = pmc_traffic("k_gbtrf_wave", ["--pmc-child", "rk3"])
+        t, why = pmc_traffic("k_gbtrf_panel", ["--pmc-child", "rk3"])
         out["roofline"]["traffic"] = t["bytes"] if t else None
         if t:
             out["roofline"]["traffic_passes"] = t["passes"]

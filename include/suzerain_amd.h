@@ -573,7 +573,8 @@ typedef struct sz_ensemble_opts {
     int nstreams;         /* explicit-stage streams (1..max_streams)        */
     int max_streams;      /* streams (and scratch sets) created, <= 8       */
     int graph;            /* capture steps in a hipGraph                    */
-    int lu_bs;            /* factorization unroll, 4 or 8 (0: 8)            */
+    int lu_bs;            /* factorization unroll, 4 or 8 (0: 8): accepted,
+                             one kernel serves both                         */
 } sz_ensemble_opts;
 sz_ensemble *sz_ensemble_create(int nmembers, const sz_channel_spec *specs,
                                 const double *dt, const sz_ensemble_opts *opts,

@@ -71,6 +71,7 @@ struct sz_ensemble {
     hipGraphExec_t exec = nullptr;
     double tuned_ms = 0;
     std::vector<double> trial_ms;         // autotune: per candidate
+    int lu_bs = 0;                        // option as given: one kernel serves all
     long long bytes = 0;
     std::vector<void *> owned;
 
@@ -328,7 +329,7 @@ sz_ensemble *sz_ensemble_create(int nmembers, const sz_channel_spec *specs,
         e->pp.tolsc = zs.tolsc();
         e->pp.reuse = zs.reuse() ? 1 : 0;
         e->pp.graph = opts->graph ? 1 : 0;
-        e->pp.lu_bs = opts->lu_bs;
+        e->lu_bs = opts->lu_bs;
         e->graph = e->pp.graph;
         e->nstreams = std::max(1, std::min(opts->nstreams, e->maxstreams));
         e->prec = sz_prec_create({}, e->pp, e->main);
@@ -526,16 +527,15 @@ int sz_ensemble_autotune(sz_ensemble *e, int steps)
     e->graph = 0;                      // trials run eagerly
     sz_prec_set_graph(e->prec, 0);
     double best = -1;
-    int best_ns = e->nstreams, best_bs = e->pp.lu_bs ? e->pp.lu_bs : 8;
+    int best_ns = e->nstreams, best_bs = e->lu_bs ? e->lu_bs : 8;
     e->trial_ms.clear();
     const int cand_ns[4] = {1, 2, 3, 4};
-    const int cand_bs[2] = {4, 8};
+    const int cand_bs[2] = {4, 8};     // one kernel: each stream count is timed twice
     for (int a = 0; a < 4 && !rc; ++a) {
         if (cand_ns[a] > e->maxstreams) continue;
         for (int b = 0; b < 2 && !rc; ++b) {
             restore();
             e->assign_streams(cand_ns[a]);
-            sz_prec_set_lu_bs(e->prec, cand_bs[b]);
             const double ms = e->trial(steps);
             e->trial_ms.push_back(ms);
             if (ms > 0 && (best < 0 || ms < best)) {
@@ -547,8 +547,7 @@ int sz_ensemble_autotune(sz_ensemble *e, int steps)
     }
     restore();
     e->assign_streams(best_ns);
-    e->pp.lu_bs = best_bs;
-    sz_prec_set_lu_bs(e->prec, best_bs);
+    e->lu_bs = best_bs;
     e->graph = graph;
     sz_prec_set_graph(e->prec, graph);
     e->tuned_ms = best;
@@ -562,7 +561,7 @@ int sz_ensemble_tuning(const sz_ensemble *e, int *nstreams, int *lu_bs,
 {
     if (!e) return -1;
     if (nstreams) *nstreams = e->nstreams;
-    if (lu_bs) *lu_bs = e->pp.lu_bs;
+    if (lu_bs) *lu_bs = e->lu_bs;
     int n = 0;
     for (double t : e->trial_ms) {
         if (trial_ms && n < max) trial_ms[n] = t;

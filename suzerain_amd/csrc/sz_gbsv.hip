@@ -17,10 +17,9 @@
 // active (kl+1) x (kl+ku+1) window of rows j..j+kl and columns j..j+kl+ku
 // stays on chip, so an elimination step brings in one row (row j+kl+1) and
 // sends out one row (U row j) and one column (the multipliers of column j).
-//   * k_gbtrf_wave: one wavefront per system, one window column per lane,
-//     the rows in registers; no barriers, about 400 VALU instructions per
-//     step (760 with the fused U^T solve).  Used for the band shapes of the
-//     channel operators.
+//   * k_gbtrf_panel: one wavefront per system, one window column per lane,
+//     the rows in registers, four columns at a time; no barriers.  Used for
+//     the band shapes of the channel operators.
 //   * k_gbtrf: one workgroup per system, the window in LDS as a circular
 //     buffer in both directions; wave 0 does the pivot search, the swap and
 //     the scaling, then all waves apply the rank-1 update.  Any band shape.
@@ -29,6 +28,10 @@
 #include <cstdlib>
 #include <type_traits>
 #include <utility>
+
+// the compiler's DPP move for 64-bit values (its builtin takes 32 bits only)
+__device__ double sz_update_dpp(double, double, int, int, int, bool)
+    __asm("llvm.amdgcn.update.dpp.f64");
 
 namespace {
 
@@ -859,71 +862,296 @@ void k_gbtrs_t16(int n, const cpx<R> *__restrict__ ab, int ldab, long long sab,
     for (int i = l; i < ns; i += LPS) sz::gstore(bs + i, x[i]);
 }
 
-// ---------------------------------------------------------------- wave
-// One wavefront per system, no barriers.  Lane l holds the window column
-// j + ((l - j) mod 64) as WR = kl+1 row slots in registers.  Steps run in
-// blocks of WV_BS, unrolled: at the start of a block slot s holds row
-// jb+s, row jb+u leaves slot u at step u and row jb+u+WR enters it, and at
-// the end of the block the slots are renamed by WV_BS so the next block
-// starts aligned again.  Every register slot index in a step is therefore a
-// compile-time constant (the rank-1 update, the pivot-column transpose, U
-// row j, the entering row, the column retire); only the pivot row of an
-// interchange is data dependent, and that path selects over the slots.
-// Columns j+64 .. j+kl+ku (kl+ku >= 64) live in an LDS tail, column j+64+t
-// in tail slot (th+t) mod NTAIL, row i at i mod WR (stored twice, so a
-// column reads back in register order from one base address).  Step j:
-//   * lane r <= km needs row j+r of column j.  At a block start the lanes
-//     holding the block's WV_BS columns write them to LDS together, one
-//     store per slot for all of them (tcol, row per slot).  Each step then
-//     applies its update to the later block columns there as well: lane r
-//     updates the row its multiplier belongs to with U(j, k) read from the
-//     lane holding column k, the same fnms the registers see, and the lanes
-//     holding those columns store the entering row; an interchange swaps
-//     the two rows there as it does in registers.  After a skipped update
-//     (zero pivot) the rest of the block falls back to the lane holding
-//     column j writing it out.  The pivot is the first lane whose
-//     |Re|+|Im| equals the DPP and readlane maximum (a NaN in row j wins,
-//     any other NaN never does);
-//   * lane r forms multiplier r (zero for row j and rows past n); the update
-//     is one static loop without predicates that takes the multiplier of
-//     slot s from its row's lane by readlane (LDS issue, not VALU, is what
-//     several waves per SIMD contend for), and lane r also writes it to LDS
-//     at row j+r's slot for the far-pivot tail path;
-//   * every lane stores U(j, its column), U(j, a tail column), L(lane, j)
-//     and the pivot index, and issues two prefetch loads, all unconditional
-//     (lanes with nothing to write store U(j,j) again), so outstanding
-//     memory operations are counted exactly.
+// --------------------------------------------------------------- panel
+// The factorization of the channel band shapes: one wavefront per system, no
+// barriers, four columns at a time.  Lane l holds window column jb + d,
+// d = (l - jb) mod 64, as PR = kl + 4 row slots in registers (slot s = row
+// jb + s); columns jb+64 .. jb+kl+ku+3 (kl+ku >= 64) live in an LDS tail.  A
+// block of four columns:
+//   1. The panel columns go through LDS into row layout: slot 16m + i in
+//      register m of the i-th lane of every 16-lane row, so each of the four
+//      DPP rows holds the whole column.  Pivot search (maximum of the high
+//      words by DPP, the low words on a tie only), interchange, multipliers
+//      and the panel's own updates run there without leaving the row.  The
+//      reciprocal's two quotients and the two of U^T's y are one division, a
+//      numerator for each lane of a quad.
+//   2. Every lane then applies the four interchanges and updates to its
+//      column.  The multiplier of a slot is a row_newbcast operand of the
+//      fused multiply-add itself: no readlane and no LDS read per multiplier
+//      (two readlanes cost as much as a multiply-add: 13.8 against 6.0 cycles
+//      for the pair, measured).
+//   3. U rows leave and the next rows enter as 64 contiguous bytes per column
+//      (one element at a time moved 2.5 times the bytes: 15.9 GB per 4560
+//      systems against 6.3 now and 6.1 needed), the rows straight to LDS
+//      early in the block so that no wait for them falls on the stores; the
+//      slots are renamed by four.
 // Every updated element sees the fnms sequence of the unblocked loop.
 //
+// What bounds it: vector issue, about 300 instructions per column step, 136
+// of them the multiply-adds of step 2 (they alone would take a fifth of the
+// time).  At two waves per SIMD (the window takes 152 of a lane's registers)
+// the pivot chain of one wave runs beside the updates of the other.  4560
+// systems of N = 480, kl = ku = 34, diagonally dominant: 2.85 ms, fused with
+// U^T 3.07 ms (an unblocked loop with readlane multipliers: 5.15 and 5.40
+// ms); 1152 systems 1.01 (1.50), one system 0.76 with U^T (1.21); complex
+// float 2.49 (5.37).
+//
 // UT = true also solves U^T y = b on the way (the first half of ZGBTRS 'T'):
-// lane l keeps the pending b of its column, y_j = b_j / U(j,j) is formed
-// when U row j is final and every lane with a column j+d, 1 <= d <= kl+ku,
-// subtracts U(j, j+d) y_j -- x_k receives its terms for ascending rows, the
-// sequential order of the LAPACK loop.  y overwrites b.
-constexpr int WV_PF = 2;
+// lane l keeps the pending b of its column, y_j = b_j / U(j,j) is formed with
+// the multipliers of column j and every lane with a column j+d, 1 <= d <=
+// kl+ku, subtracts U(j, j+d) y_j -- x_k receives its terms for ascending
+// rows, the sequential order of the LAPACK loop.  y overwrites b.
+constexpr int PN_NB = 4;
 
-template <typename R, int WR, int KV, int WV_BS, bool UT = false>
-__global__ __launch_bounds__(64)
-void k_gbtrf_wave(int n, cpx<R> *__restrict__ ab, int ldab, long long sab,
-                  int *__restrict__ ipiv, long long sipiv,
-                  int *__restrict__ info, const int *__restrict__ skip,
-                  int nsys, cpx<R> *__restrict__ bv = nullptr, long long sb = 0,
-                  int prio = 0, const sz::gsys *__restrict__ gs = nullptr)
+// Waves per SIMD.  The window takes 152 (34 sub-diagonals) or 112 (24) of a
+// lane's registers in double precision, so three waves fit only the narrower
+// shape without U^T (fused they spill: 2.89 ms per 4560 systems of N = 365
+// against 1.79).  Single precision would fit four, but runs faster with two
+// (12,000 systems of N = 960: 11.7 ms against 13.1 with three and 13.5 with
+// four; 4560 of N = 480: 2.49, 2.63, 2.72): a visit takes 32 bytes of a
+// column's cache line, and more systems at once push the lines out of the L2
+// between visits.
+constexpr int panel_waves(size_t real, int wr, bool ut)
+{
+    return real == 8 && wr <= 25 && !ut ? 3 : 2;
+}
+
+// v of lane S of each 16-lane row, in every lane of that row
+template <int S, typename R>
+__device__ __forceinline__ R row_bcast(R v)
+{
+    if constexpr (sizeof(R) == 8)
+        return sz_update_dpp(0.0, v, 0x150 + S, 0xF, 0xF, true);
+    else
+        return __builtin_bit_cast(
+            R, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + S, 0xF,
+                                           0xF, true));
+}
+
+// a_i -= l[lane L0 + i] u for i < N (N = 1 or 4), l read from lanes L0 .. of
+// the same 16-lane row: the two nested multiply-adds of sz::cfnms.  Written
+// as instructions because the compiler does not fold a 64-bit row broadcast
+// into the multiply-add; the leading s_nop covers the two wait states a DPP
+// operand needs after the instruction that wrote it.
+template <int L0, typename R>
+__device__ __forceinline__ void fnms_row1(R &ax, R &ay, R lx, R ly, R ux, R uy)
+{
+    if constexpr (sizeof(R) == 8)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, -%2, %4 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, -%2, %5 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %0, %3, %5 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, -%3, %4 row_newbcast:%c6 row_mask:0xf bank_mask:0xf"
+            : "+v"(ax), "+v"(ay) : "v"(lx), "v"(ly), "v"(ux), "v"(uy), "n"(L0));
+    else
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, -%2, %4 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, -%2, %5 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %0, %3, %5 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, -%3, %4 row_newbcast:%c6 row_mask:0xf bank_mask:0xf"
+            : "+v"(ax), "+v"(ay) : "v"(lx), "v"(ly), "v"(ux), "v"(uy), "n"(L0));
+}
+#define PN_LINE(OP, A, L, U, C) OP " %" #A ", " L ", %" #U " row_newbcast:%c" #C         \
+                                " row_mask:0xf bank_mask:0xf\n\t"
+#define PN_FOUR(OP)                                                             \
+    "s_nop 1\n\t"                                                               \
+    PN_LINE(OP, 0, "-%8", 10, 12) PN_LINE(OP, 1, "-%8", 11, 12)                   \
+    PN_LINE(OP, 2, "-%8", 10, 13) PN_LINE(OP, 3, "-%8", 11, 13)                   \
+    PN_LINE(OP, 4, "-%8", 10, 14) PN_LINE(OP, 5, "-%8", 11, 14)                   \
+    PN_LINE(OP, 6, "-%8", 10, 15) PN_LINE(OP, 7, "-%8", 11, 15)                   \
+    PN_LINE(OP, 0, "%9", 11, 12) PN_LINE(OP, 1, "-%9", 10, 12)                    \
+    PN_LINE(OP, 2, "%9", 11, 13) PN_LINE(OP, 3, "-%9", 10, 13)                    \
+    PN_LINE(OP, 4, "%9", 11, 14) PN_LINE(OP, 5, "-%9", 10, 14)                    \
+    PN_LINE(OP, 6, "%9", 11, 15) PN_LINE(OP, 7, "-%9", 10, 15)
+template <int L0, typename R>
+__device__ __forceinline__ void fnms_row4(R &ax0, R &ay0, R &ax1, R &ay1, R &ax2, R &ay2,
+                                          R &ax3, R &ay3, R lx, R ly, R ux, R uy)
+{
+    if constexpr (sizeof(R) == 8)
+        asm(PN_FOUR("v_fmac_f64_dpp")
+            : "+v"(ax0), "+v"(ay0), "+v"(ax1), "+v"(ay1), "+v"(ax2), "+v"(ay2),
+              "+v"(ax3), "+v"(ay3)
+            : "v"(lx), "v"(ly), "v"(ux), "v"(uy), "n"(L0), "n"(L0 + 1), "n"(L0 + 2),
+              "n"(L0 + 3));
+    else
+        asm(PN_FOUR("v_fmac_f32_dpp")
+            : "+v"(ax0), "+v"(ay0), "+v"(ax1), "+v"(ay1), "+v"(ax2), "+v"(ay2),
+              "+v"(ax3), "+v"(ay3)
+            : "v"(lx), "v"(ly), "v"(ux), "v"(uy), "n"(L0), "n"(L0 + 1), "n"(L0 + 2),
+              "n"(L0 + 3));
+}
+#undef PN_FOUR
+#undef PN_LINE
+
+template <int... I, typename F>
+__device__ __forceinline__ void unroll_impl(F &&f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int K, typename F>
+__device__ __forceinline__ void unroll(F &&f)
+{
+    unroll_impl(f, std::make_integer_sequence<int, K>{});
+}
+
+// One element per lane from p (64 lanes) straight to LDS at dst, without
+// passing through registers: complex doubles as they are, complex floats as
+// a run of the real parts and a run of the imaginary ones (a transfer moves
+// 4 or 16 bytes a lane).  take_lds reads a lane's own element back.
+template <typename R>
+__device__ __forceinline__ void load_lds(const cpx<R> *p, cpx<R> *dst)
+{
+    using G = const __attribute__((address_space(1))) unsigned;
+    using L = __attribute__((address_space(3))) unsigned;
+    if constexpr (sizeof(R) == 8) {
+        __builtin_amdgcn_global_load_lds((G *)(p), (L *)(dst), 16, 0, 0);
+    } else {
+        __builtin_amdgcn_global_load_lds((G *)(p), (L *)(dst), 4, 0, 0);
+        __builtin_amdgcn_global_load_lds((G *)(&p->y), (L *)(dst + 32), 4, 0, 0);
+    }
+}
+
+template <typename R>
+__device__ __forceinline__ void take_lds(const cpx<R> *src, int lane, R &x, R &y)
+{
+    const R *v = reinterpret_cast<const R *>(src);
+    x = v[sizeof(R) == 8 ? 2 * lane : lane];
+    y = v[sizeof(R) == 8 ? 2 * lane + 1 : 64 + lane];
+}
+
+// c ? a : b by value (a conditional between array elements is a choice of
+// addresses, which can keep the arrays in scratch memory)
+template <typename R>
+__device__ __forceinline__ R pick(bool c, R a, R b) { return c ? a : b; }
+
+template <typename R>
+__device__ __forceinline__ R pick4(int k, R a, R b, R c, R e)
+{
+    return pick(k == 0, a, pick(k == 1, b, pick(k == 2, c, e)));
+}
+
+// slots S .. S1 of the window receive one update: four at a time from
+// aligned slots, one at a time at the ends
+template <int S, int S1, typename R, int PR, int NM>
+__device__ __forceinline__ void panel_update(R (&ax)[PR], R (&ay)[PR], const R (&lx)[NM],
+                                             const R (&ly)[NM], R ux, R uy)
+{
+    if constexpr (S <= S1) {
+        if constexpr (S % 4 == 0 && S + 3 <= S1) {
+            fnms_row4<S % 16>(ax[S], ay[S], ax[S + 1], ay[S + 1], ax[S + 2], ay[S + 2],
+                              ax[S + 3], ay[S + 3], lx[S / 16], ly[S / 16], ux, uy);
+            panel_update<S + 4, S1>(ax, ay, lx, ly, ux, uy);
+        } else {
+            fnms_row1<S % 16>(ax[S], ay[S], lx[S / 16], ly[S / 16], ux, uy);
+            panel_update<S + 1, S1>(ax, ay, lx, ly, ux, uy);
+        }
+    }
+}
+
+// a[U] <-> a[sp] in the lanes of `in`; sp (uniform) in U+1 .. LAST.  The
+// branch to the slot is inside the instructions: as branches of the source
+// the exchanges are merged into one that indexes the window at run time, in
+// scratch memory, or copy the window at every join.
+#define PN_SWAP64(A, B)                                                         \
+    "v_mov_b64 %[t], %[" A "]\n\tv_mov_b64 %[" A "], %[" B "]\n\t"              \
+    "v_mov_b64 %[" B "], %[t]\n\t"
+#define PN_SWAP32(A, B) "v_swap_b32 %[" A "], %[" B "]\n\t"
+#define PN_ONE(SW, I)                                                           \
+    "s_cmp_lg_u32 %[sp], %c[s" I "]\n\ts_cbranch_scc1 .Lpn" I "_%=\n\t"         \
+    SW("ux", "x" I) SW("uy", "y" I) ".Lpn" I "_%=:\n\t"
+#define PN_GROUP(SW)                                                            \
+    "s_lshr_b32 %[g], %[sp], 2\n\ts_cmp_lg_u32 %[g], %c[grp]\n\t"               \
+    "s_cbranch_scc1 .Lpn4_%=\n\ts_and_saveexec_b64 %[save], %[in]\n\t"          \
+    PN_ONE(SW, "0") PN_ONE(SW, "1") PN_ONE(SW, "2") PN_ONE(SW, "3")             \
+    "s_mov_b64 exec, %[save]\n\t.Lpn4_%=:"
+template <int U, int S, int LAST, typename R, int PR>
+__device__ __forceinline__ void slot_swap(R (&ax)[PR], R (&ay)[PR], int sp,
+                                          unsigned long long in)
+{
+    if constexpr (S <= LAST) {
+        // slots S .. S+3; in place of slot U itself or a slot past the window
+        // (never sp) a spare register
+        R nx[4], ny[4], t;
+        unroll<4>([&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value, q = S + i;
+            if constexpr (q > U && q < PR) {
+                nx[i] = ax[q];
+                ny[i] = ay[q];
+            } else {
+                nx[i] = ny[i] = R(0);
+            }
+        });
+        unsigned g;
+        unsigned long long save;
+#define PN_OPERANDS                                                             \
+        : [ux] "+v"(ax[U]), [uy] "+v"(ay[U]), [x0] "+v"(nx[0]), [y0] "+v"(ny[0]), \
+          [x1] "+v"(nx[1]), [y1] "+v"(ny[1]), [x2] "+v"(nx[2]), [y2] "+v"(ny[2]), \
+          [x3] "+v"(nx[3]), [y3] "+v"(ny[3]), [t] "=&v"(t), [g] "=&s"(g),        \
+          [save] "=&s"(save)                                                    \
+        : [sp] "s"(sp), [in] "s"(in), [grp] "n"(S / 4), [s0] "n"(S), [s1] "n"(S + 1), \
+          [s2] "n"(S + 2), [s3] "n"(S + 3)                                      \
+        : "scc"
+        if constexpr (sizeof(R) == 8) asm volatile(PN_GROUP(PN_SWAP64) PN_OPERANDS);
+        else asm volatile(PN_GROUP(PN_SWAP32) PN_OPERANDS);
+#undef PN_OPERANDS
+        unroll<4>([&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value, q = S + i;
+            if constexpr (q > U && q < PR) {
+                ax[q] = nx[i];
+                ay[q] = ny[i];
+            }
+        });
+        slot_swap<U, S + 4, LAST>(ax, ay, sp, in);
+    }
+}
+#undef PN_GROUP
+#undef PN_ONE
+#undef PN_SWAP32
+#undef PN_SWAP64
+
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp_max(unsigned v)
+{
+    const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+    return v > o ? v : o;
+}
+
+// maximum over the 16 lanes of a row, in every lane of it
+__device__ __forceinline__ unsigned row_max16(unsigned v)
+{
+    v = dpp_max<0xB1>(v);                    // quad_perm [1,0,3,2]
+    v = dpp_max<0x4E>(v);                    // quad_perm [2,3,0,1]
+    v = dpp_max<0x124>(v);                   // row_ror:4
+    return dpp_max<0x128>(v);                // row_ror:8
+}
+
+// words of a nonnegative number, ordered as the number is: the high word
+// (all of a float) and the low word
+__device__ __forceinline__ unsigned key_hi(double v) { return (unsigned)__double2hiint(v); }
+__device__ __forceinline__ unsigned key_lo(double v) { return (unsigned)__double2loint(v); }
+__device__ __forceinline__ unsigned key_hi(float v) { return __builtin_bit_cast(unsigned, v); }
+__device__ __forceinline__ unsigned key_lo(float) { return 0; }
+
+template <typename R, int WR, int KV, bool UT, int WPE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+void k_gbtrf_panel(int n, cpx<R> *__restrict__ ab, int ldab, long long sab,
+                   int *__restrict__ ipiv, long long sipiv, int *__restrict__ info,
+                   const int *__restrict__ skip, int nsys, cpx<R> *__restrict__ bv,
+                   long long sb, const sz::gsys *__restrict__ gs)
 {
     using T = cpx<R>;
-    constexpr int kl = WR - 1, ku = KV - kl;
-    constexpr int NTAIL = KV >= 64 ? KV - 63 : 0;
-    constexpr int TW = 2 * WR;                     // tail column stride
-    static_assert(WR > WV_BS && WR <= 40 && WV_BS % WV_PF == 0, "row slots");
-    static_assert(KV <= 127 && ku >= 0, "window");
-    __shared__ T colbuf[WR];
-    __shared__ T lbuf[WR];
-    // the row-per-slot block columns pay off when LDS is the shared limit,
-    // i.e. with several waves per SIMD: the fused solve of the full batch
-    constexpr bool TCOL = UT;
-    __shared__ T tcol[TCOL ? WV_BS : 1][WR];       // block columns, row per slot
-    __shared__ T tail[NTAIL > 0 ? NTAIL * TW : 1];
-    __shared__ T tailb[NTAIL > 0 ? NTAIL : 1];     // pending b of tail columns
+    constexpr int NB = PN_NB, kl = WR - 1, ku = KV - kl;
+    constexpr int PR = kl + NB;                    // rows of a block's window
+    constexpr int NM = (PR + 15) / 16;             // registers of a panel column
+    constexpr int NT = KV + NB > 64 ? KV + NB - 64 : 0;   // tail columns
+    constexpr int PS = 16 * NM + 1;                // panel column stride in LDS
+    constexpr unsigned INFW = sizeof(R) == 8 ? 0x7FF00000u : 0x7F800000u;
+    static_assert(kl >= NB && ku >= NB, "interchanges reach every panel column");
+    static_assert(NT == 0 || NT == 2 * NB, "tail");
+    __shared__ T pbuf[NB * PS];
+    __shared__ T qbuf[(NB + 2) * 64];              // what the next block needs
+    __shared__ T tail[NT > 0 ? NT * PR : 1];
+    __shared__ T tailb[NT > 0 ? NT : 1];
 
     const int sys = blockIdx.x;
     if (sys >= nsys) return;
@@ -939,381 +1167,497 @@ void k_gbtrf_wave(int n, cpx<R> *__restrict__ ab, int ldab, long long sab,
         ipiv += (size_t)sys * (size_t)sipiv;
         if constexpr (UT) bv += (size_t)sys * (size_t)sb;
     }
-    const int lane = threadIdx.x;
+    int lane = threadIdx.x;
 
-    // c ? x : 0, component-wise (a select of whole structs goes through
-    // memory; literal zeros: a zero struct kept live gets spilled)
-    auto sel0 = [](bool c, T x) __attribute__((always_inline)) -> T {
-        T o;
-        o.x = c ? x.x : R(0);
-        o.y = c ? x.y : R(0);
-        return o;
-    };
     auto band = [&](int i, int c) __attribute__((always_inline)) -> T {
         const bool ok = i < n && c < n && c - i <= ku && i - c <= kl;
-        const auto p = sz::gmem(ab + (ok ? (size_t)c * ldab + KV + i - c : 0));
-        const R x = p->x, y = p->y;
-        return T{ok ? x : R(0), ok ? y : R(0)};
-    };
-    // raw element (clamped address; validity is applied when consumed)
-    auto raw = [&](int i, int c) __attribute__((always_inline)) -> T {
-        const bool ok = i < n && c < n;
-        return sz::gload(ab + (ok ? (size_t)c * ldab + KV + i - c : 0));
+        const T v = sz::gload(ab + (ok ? (size_t)c * ldab + KV + i - c : 0));
+        return T{ok ? v.x : R(0), ok ? v.y : R(0)};
     };
 
-    T a[WR];
-#pragma unroll
-    for (int s = 0; s < WR; ++s) a[s] = band(s, lane);
-    if constexpr (NTAIL > 0) {
-        for (int e = lane; e < NTAIL * WR; e += 64) {
-            const int t = e / WR, p = e - t * WR;
-            const T v = band(p, 64 + t);
-            tail[t * TW + p] = v;
-            tail[t * TW + p + WR] = v;
+    // component arrays throughout: arrays of structs go through scratch
+    R ax[PR], ay[PR];
+    unroll<PR>([&](auto s_) __attribute__((always_inline)) {
+        constexpr int s = decltype(s_)::value;
+        const T v = band(s, lane);
+        ax[s] = v.x;
+        ay[s] = v.y;
+    });
+    if constexpr (NT > 0) {
+        for (int e = lane; e < NT * PR; e += 64) {
+            const int t = e / PR;
+            tail[e] = band(e - t * PR, 64 + t);
         }
     }
-    // entering row u+WR: this lane's column after step u, and tail column
-    // u+65+lane
-    T qv[WV_PF], qt[WV_PF];
-#pragma unroll
-    for (int u = 0; u < WV_PF; ++u) {
-        qv[u] = raw(u + WR, u + 1 + ((lane - (u + 1)) & 63));
-        qt[u] = raw(u + WR, lane < NTAIL ? u + 65 + lane : n);
-    }
-    // U^T solve: the pending b of this lane's column and, prefetched, the b
-    // of the column that enters the window at each step (uniform address)
-    constexpr int BNEW = NTAIL > 0 ? KV + 1 : 64;   // column j+BNEW enters at step j
-    T breg{R(0), R(0)}, qb[WV_PF];
+    for (int e = lane; e < NB * PS; e += 64) pbuf[e] = T{R(0), R(0)};
+    R bx = R(0), by = R(0);
     if constexpr (UT) {
-        breg = sel0(lane < n, sz::gload(bv + (lane < n ? lane : 0)));
-        if (NTAIL > 0 && lane < NTAIL) {
-            tailb[lane] = sel0(64 + lane < n, sz::gload(bv + (64 + lane < n ? 64 + lane : 0)));
+        const T v = sz::gload(bv + (lane < n ? lane : 0));
+        bx = lane < n ? v.x : R(0);
+        by = lane < n ? v.y : R(0);
+        if (NT > 0 && lane < NT) {
+            const int c = 64 + lane;
+            const T w = sz::gload(bv + (c < n ? c : 0));
+            tailb[lane] = T{c < n ? w.x : R(0), c < n ? w.y : R(0)};
         }
-#pragma unroll
-        for (int u = 0; u < WV_PF; ++u) qb[u] = sz::gload(bv + min(u + BNEW, n - 1));
     }
     WAVE_SYNC();
 
-    int c0 = 0, th = 0, ju = 0, first_zero = 0;
-    int ob = 0;                                      // jb mod WR
-    const int lane_id = lane;
-    for (int jb = 0; jb < n; jb += WV_BS) {
-        bool replay = TCOL;                          // tcol is current
-#pragma unroll
-        for (int u = 0; u < WV_BS; ++u) {
-            if (jb + u >= n) break;
-            // recompute step-derived values each step: hoisted out of the
-            // unrolled steps they become per-step induction variables and
-            // 64-bit lane masks that overflow the scalar registers (101
-            // spilled to VGPR lanes, 54 with these barriers)
-            int j = jb + u;
-            asm volatile("" : "+s"(j), "+s"(c0), "+s"(th), "+s"(ob));
-            int lane = lane_id;
-            asm volatile("" : "+v"(lane));
-            // with more systems than SIMDs but fewer than two per SIMD, the
-            // SIMDs holding two waves finish last: there the wave in its
-            // pivot chain issues ahead of the other's rank-1 update (the
-            // fused kernel runs the 4560-system substep batch, where the
-            // test alone costs 2%)
-            if constexpr (!UT)
-                if (prio) __builtin_amdgcn_s_setprio(3);
-            const int j0 = ob + u >= WR ? ob + u - WR : ob + u;   // j mod WR
-            const int km = min(kl, n - 1 - j);
-            const int d = (lane - c0) & 63;          // this lane: column j + d
-            const size_t ujj = (size_t)j * ldab + KV;
-
-            // ---- column j, row j+lane in lane (slot s holds row jb+s at u = 0)
-            if (TCOL && u == 0) {
-                if (d < WV_BS) {
-#pragma unroll
-                    for (int s = 0; s < WR; ++s) tcol[d][s] = a[s];
-                }
-            } else if (!replay && d == 0) {
-#pragma unroll
-                for (int s = 0; s < WR; ++s) colbuf[s] = a[s];
+    int first_zero = 0, ju = 0;
+    for (int jb = 0; jb < n; jb += NB) {
+        // what follows from the lane is recomputed in every block: held
+        // through the loop it would not fit the registers
+        asm volatile("" : "+v"(lane));
+        const int l16 = lane & 15, lq = lane & 3;
+        const int c0 = jb & 63;
+        // ---- 1. panel columns (lanes with column jb + d, d < NB) to row layout
+        if (((lane - c0) & 63) < NB) {
+            T *dst = pbuf + ((lane - c0) & 63) * PS;
+            unroll<PR>([&](auto s_) __attribute__((always_inline)) {
+                constexpr int s = decltype(s_)::value;
+                dst[s] = T{ax[s], ay[s]};
+            });
+        }
+        // rows jb+PR .. jb+PR+3 of the next block's columns (of the tail's:
+        // column lane/4, row lane%4) and the b of the columns it brings in,
+        // straight to LDS: they arrive during the panel and the updates, and
+        // registers to hold them are not to be had
+        {
+            const int cn = jb + NB + ((lane - c0 - NB) & 63);
+            const T *src = ab + (cn < n ? (size_t)cn * ldab + KV + jb + PR - cn : 0);
+            unroll<NB>([&](auto i_) __attribute__((always_inline)) {
+                constexpr int i = decltype(i_)::value;
+                load_lds(cn < n && jb + PR + i < n ? src + i : ab, &qbuf[i * 64]);
+            });
+            if constexpr (NT > 0) {
+                const int c = jb + NB + 64 + (lane >> 2), r = jb + PR + lq;
+                load_lds(ab + (lane < NT * NB && c < n && r < n
+                                   ? (size_t)c * ldab + KV + r - c : 0), &qbuf[NB * 64]);
             }
-            WAVE_SYNC();
-            int ps = u + lane;                        // slot of row j+lane
-            if (ps >= WR) ps -= WR;
-            const T v = sel0(lane < WR, replay ? tcol[u][lane < WR ? ps : 0]
-                                               : colbuf[lane < WR ? ps : 0]);
-            R key = R(-1);
-            {
-                const R m1 = fabs(v.x) + fabs(v.y);
-                if (lane <= km) key = (m1 != m1) ? (lane == 0 ? R(__builtin_inff()) : R(-1)) : m1;
-            }
-            R m = key;
-            m = fmax(m, dpp_r<0xB1>(m));             // quad_perm [1,0,3,2]
-            m = fmax(m, dpp_r<0x4E>(m));             // quad_perm [2,3,0,1]
-            m = fmax(m, dpp_r<0x124>(m));            // row_ror:4
-            m = fmax(m, dpp_r<0x128>(m));            // row_ror:8
-            const R mx = fmax(fmax(readlane_r(m, 0), readlane_r(m, 16)),
-                              fmax(readlane_r(m, 32), readlane_r(m, 48)));
-            const unsigned long long ball = __ballot(key == mx);
-            const int jp = (int)__builtin_ctzll(ball);
-            T piv, v0;
-            piv.x = readlane_r(v.x, jp);
-            piv.y = readlane_r(v.y, jp);
-            v0.x = readlane_r(v.x, 0);
-            v0.y = readlane_r(v.y, 0);
-            const bool nz = sz::cnonzero(piv);
-            if (nz) ju = max(ju, min(j + ku + jp, n - 1));
-            else if (first_zero == 0) first_zero = j + 1;
-            *sz::gmem(ipiv + j) = j + jp + 1;
-
-            // ---- multipliers (row jp now holds old row j)
-            T l = v;
-            if (nz) {
-                const T rcp = sz::crcp(piv);
-                T w = v;
-                if (lane == jp) w = v0;
-                l = sz::cmul(w, rcp);
-            }
-            const bool isl = lane >= 1 && lane <= km;
-            T lz = sel0(isl, l);
-            // the update below runs under a divergent mask and reads every
-            // lane's multiplier by readlane: pin it here, where all lanes are
-            // active, so it is not computed inside the mask instead
-            asm volatile("" : "+v"(lz.x), "+v"(lz.y));
-            if (lane < WR) lbuf[ps] = lz;
-            {
-                T st;
-                st.x = isl ? l.x : piv.x;
-                st.y = isl ? l.y : piv.y;
-                sz::gstore(ab + (isl ? ujj + lane : ujj), st);
-            }
-
-            // ---- interchange rows j and j+jp in columns j .. ju
-            T uc = a[u];
-            if (nz && jp != 0) {
-                const bool inr = d <= ju - j;
-                const int sp = u + jp >= WR ? u + jp - WR : u + jp;
-                T rp = uc;
-#pragma unroll
-                for (int s = 0; s < WR; ++s) {
-                    if (s != u) {
-                        rp.x = s == sp ? a[s].x : rp.x;
-                        rp.y = s == sp ? a[s].y : rp.y;
-                        a[s].x = (s == sp && inr) ? uc.x : a[s].x;
-                        a[s].y = (s == sp && inr) ? uc.y : a[s].y;
-                    }
-                }
-                uc.x = inr ? rp.x : uc.x;
-                uc.y = inr ? rp.y : uc.y;
-                a[u] = uc;
-                if constexpr (NTAIL > 0) {
-                    if (ju >= j + 64 && lane < NTAIL && j + 64 + lane <= ju) {
-                        const int pp = j0 + jp >= WR ? j0 + jp - WR : j0 + jp;
-                        int ts = th + lane;
-                        if (ts >= NTAIL) ts -= NTAIL;
-                        // component-wise: struct copies here go through
-                        // scratch memory
-                        R *tc = reinterpret_cast<R *>(tail + ts * TW);
-                        const R t0x = tc[2 * j0], t0y = tc[2 * j0 + 1];
-                        const R t1x = tc[2 * pp], t1y = tc[2 * pp + 1];
-                        tc[2 * j0] = t1x;
-                        tc[2 * j0 + 1] = t1y;
-                        tc[2 * (j0 + WR)] = t1x;
-                        tc[2 * (j0 + WR) + 1] = t1y;
-                        tc[2 * pp] = t0x;
-                        tc[2 * pp + 1] = t0y;
-                        tc[2 * (pp + WR)] = t0x;
-                        tc[2 * (pp + WR) + 1] = t0y;
-                    }
-                }
-            }
-            // the block's later columns, row per slot, receive this step's
-            // update as their registers do (same multiplier, same U(j, k),
-            // same fnms) unless a skipped update ends that
-            if (!nz || km == 0) replay = false;
-            if (replay) {
-                // an interchange of rows j and j+jp reaches the block columns
-                // too (they lie within ju): rows j and j+jp read each other's
-                // slot before the update
-                int src = ps;
-                if (nz && jp != 0) {
-                    const int sp = u + jp >= WR ? u + jp - WR : u + jp;
-                    src = lane == 0 ? sp : (lane == jp ? u : ps);
-                }
-#pragma unroll
-                for (int k = u + 1; k < WV_BS; ++k) {
-                    T uk;
-                    uk.x = readlane_r(uc.x, (c0 + k - u) & 63);
-                    uk.y = readlane_r(uc.y, (c0 + k - u) & 63);
-                    if (lane < WR) {
-                        const T t = tcol[k][src];
-                        tcol[k][ps] = sz::cfnms(t, lz, uk);
-                    }
-                }
-            }
-            WAVE_SYNC();
-
-            // ---- U row j
-            {
-                const int cg = j + d;
-                const bool ok = d > 0 && d <= KV && cg < n;
-                T st;
-                st.x = ok ? uc.x : piv.x;
-                st.y = ok ? uc.y : piv.y;
-                sz::gstore(ab + (ok ? (size_t)cg * ldab + KV - d : ujj), st);
-            }
-            if constexpr (NTAIL > 0) {
-                int ts = th + lane;
-                if (ts >= NTAIL) ts -= NTAIL;
-                const bool ok = lane < NTAIL && j + 64 + lane < n;
-                const T tv = tail[(lane < NTAIL ? ts : 0) * TW + j0];
-                T st;
-                st.x = ok ? tv.x : piv.x;
-                st.y = ok ? tv.y : piv.y;
-                sz::gstore(ab + (ok ? (size_t)(j + 64 + lane) * ldab + KV - 64 - lane : ujj), st);
-            }
-
-            // ---- U^T solve: y_j, then U(j, j+d) y_j out of every pending b
             if constexpr (UT) {
-                T bj;
-                bj.x = readlane_r(breg.x, c0);
-                bj.y = readlane_r(breg.y, c0);
-                const T y = sz::cdiv(bj, piv);       // U(j, j) = piv
-                sz::gstore(bv + j, y);
-                if (d >= 1 && d <= KV) breg = sz::cfnms(breg, uc, y);
-                if constexpr (NTAIL > 0) {
-                    if (lane < NTAIL && j + 64 + lane < n) {
-                        int ts = th + lane;
-                        if (ts >= NTAIL) ts -= NTAIL;
-                        const T tv = tail[ts * TW + j0];
-                        tailb[ts] = sz::cfnms(tailb[ts], tv, y);
+                const int c = jb + 64 + (NT > 0 ? NB + lane : (lane - c0) & 63);
+                load_lds(bv + (c < n ? c : 0), &qbuf[(NB + 1) * 64]);
+            }
+        }
+        WAVE_SYNC();
+        R px[NB][NM], py[NB][NM];
+        unroll<NB>([&](auto k_) __attribute__((always_inline)) {
+            constexpr int k = decltype(k_)::value;
+            unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                constexpr int m = decltype(m_)::value;
+                const T v = pbuf[k * PS + 16 * m + l16];
+                px[k][m] = v.x;
+                py[k][m] = v.y;
+            });
+        });
+        R bkx[NB], bky[NB], yx[NB], yy[NB];
+        if constexpr (UT) {
+            unroll<NB>([&](auto k_) __attribute__((always_inline)) {
+                constexpr int k = decltype(k_)::value;
+                bkx[k] = readlane_r(bx, c0 + k);
+                bky[k] = readlane_r(by, c0 + k);
+            });
+        }
+        int jp[NB], jus[NB];
+        unsigned nz = 0, odd = 0;                  // bit u: step u's
+        unroll<NB>([&](auto uc_) __attribute__((always_inline)) {
+            constexpr int u = decltype(uc_)::value;
+            const int j = jb + u;
+            const int km = min(kl, n - 1 - j);     // negative past the last column
+            jp[u] = 0;
+            yx[u] = yy[u] = R(0);
+            if (j < n) {
+                // the first row of the largest |Re|+|Im|; a NaN in row j wins,
+                // any other NaN never does
+                unsigned kh[NM], kw[NM], mx = 0, raw = 0;
+                unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                    constexpr int m = decltype(m_)::value;
+                    const int slot = 16 * m + l16;
+                    const R m1 = fabs(px[u][m]) + fabs(py[u][m]);
+                    unsigned h = key_hi(m1), w = key_lo(m1);
+                    raw = max(raw, h);
+                    const bool nan = m1 != m1;
+                    bool ok = slot <= u + km && !(nan && slot != u);
+                    if (m == 0) ok = ok && slot >= u;
+                    h = nan ? INFW : h;
+                    w = nan ? 0u : w;
+                    kh[m] = ok ? h + 1 : 0u;
+                    kw[m] = w;
+                    mx = max(mx, kh[m]);
+                });
+                mx = row_max16(mx);
+                auto first = [&](auto &&is) __attribute__((always_inline)) {
+                    unsigned long long b = 0;
+                    unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                        constexpr int m = decltype(m_)::value;
+                        b |= (__ballot(is(m)) & 0xFFFFull) << (16 * m);
+                    });
+                    return b;
+                };
+                unsigned long long at = first([&](int m) { return kh[m] == mx; });
+                if (sizeof(R) == 8 && (at & (at - 1)) != 0) {    // equal high words
+                    unsigned ml = 0;
+                    unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                        constexpr int m = decltype(m_)::value;
+                        ml = max(ml, kh[m] == mx ? kw[m] : 0u);
+                    });
+                    ml = row_max16(ml);
+                    at = first([&](int m) { return kh[m] == mx && kw[m] == ml; });
+                }
+                const int t = (int)__builtin_ctzll(at);
+                jp[u] = t - u;
+                if (jp[u] != 0) {                  // then the pivot is not zero
+                    const int tm = t >> 4, tl = t & 15;
+                    unroll<NB - u>([&](auto k_) __attribute__((always_inline)) {
+                        constexpr int k = u + decltype(k_)::value;
+                        R vx = px[k][0], vy = py[k][0];
+                        const R jx = readlane_r(vx, u), jy = readlane_r(vy, u);
+                        unroll<NM - 1>([&](auto m_) __attribute__((always_inline)) {
+                            constexpr int m = 1 + decltype(m_)::value;
+                            vx = pick(tm == m, px[k][m], vx);
+                            vy = pick(tm == m, py[k][m], vy);
+                        });
+                        const R tx = readlane_r(vx, tl), ty = readlane_r(vy, tl);
+                        unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                            constexpr int m = decltype(m_)::value;
+                            const bool here = tm == m && l16 == tl;
+                            px[k][m] = pick(here, jx, px[k][m]);
+                            py[k][m] = pick(here, jy, py[k][m]);
+                        });
+                        px[k][0] = pick(l16 == u, tx, px[k][0]);
+                        py[k][0] = pick(l16 == u, ty, py[k][0]);
+                    });
+                }
+                T piv;
+                piv.x = row_bcast<u>(px[u][0]);
+                piv.y = row_bcast<u>(py[u][0]);
+                const bool pz = __ballot(sz::cnonzero(piv)) != 0;
+                nz |= pz ? 1u << u : 0u;
+                if (pz) ju = max(ju, min(j + ku + jp[u], n - 1));
+                else if (first_zero == 0) first_zero = j + 1;
+
+                // sz::crcp of the pivot and y = sz::cdiv(b_j, pivot): Smith's
+                // quotients have one denominator, so lane lq of a quad divides
+                // the numerator of (1/z).x, (1/z).y, y.x or y.y
+                const bool big = fabs(piv.x) >= fabs(piv.y);
+                const R P = big ? piv.x : piv.y, Q = big ? piv.y : piv.x;
+                const R r = Q / P, den = P + Q * r;
+                R num = lq & 1 ? (big ? -r : R(-1)) : (big ? R(1) : r);
+                if constexpr (UT) {
+                    const R A = pick(big, bkx[u], bky[u]), B = pick(big, bky[u], bkx[u]);
+                    const R n2 = A + B * r, n3 = B - A * r;
+                    const R ny = lq & 1 ? (big ? n3 : -n3) : n2;
+                    num = lq & 2 ? ny : num;
+                }
+                const R quo = num / den;
+                const T rcp{dpp_r<0x00>(quo), dpp_r<0x55>(quo)};
+                if constexpr (UT) {
+                    yx[u] = readlane_r(quo, 2);
+                    yy[u] = readlane_r(quo, 3);
+                }
+                if (pz) {
+                    unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                        constexpr int m = decltype(m_)::value;
+                        const T l = sz::cmul(T{px[u][m], py[u][m]}, rcp);
+                        const bool below = m > 0 || l16 > u;
+                        px[u][m] = pick(below, l.x, px[u][m]);
+                        py[u][m] = pick(below, l.y, py[u][m]);
+                    });
+                    // a column with an infinity or NaN, or an overflowing
+                    // reciprocal: its update spares the columns beyond ju
+                    odd |= __ballot(raw >= INFW || key_hi(fabs(rcp.x)) >= INFW ||
+                                    key_hi(fabs(rcp.y)) >= INFW) != 0 ? 1u << u : 0u;
+                }
+                // the panel's later columns, rows j+1 .. j+kl
+                unroll<NB - (u + 1)>([&](auto k_) __attribute__((always_inline)) {
+                    constexpr int k = u + 1 + decltype(k_)::value;
+                    T uk;
+                    uk.x = row_bcast<u>(px[k][0]);
+                    uk.y = row_bcast<u>(py[k][0]);
+                    if (pz) {
+                        unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                            constexpr int m = decltype(m_)::value;
+                            const T v = sz::cfnms(T{px[k][m], py[k][m]},
+                                                  T{px[u][m], py[u][m]}, uk);
+                            const bool in = (m > 0 || l16 > u) &&
+                                            (16 * m + 15 <= u + kl || 16 * m + l16 <= u + kl);
+                            px[k][m] = pick(in, v.x, px[k][m]);
+                            py[k][m] = pick(in, v.y, py[k][m]);
+                        });
+                    }
+                    if constexpr (UT) {
+                        const T v = sz::cfnms(T{bkx[k], bky[k]}, uk, T{yx[u], yy[u]});
+                        bkx[k] = v.x;
+                        bky[k] = v.y;
+                    }
+                });
+            }
+            jus[u] = ju - jb;                      // last column of the update, as d
+        });
+
+        asm volatile("" : "+v"(lane));
+        // the panel columns are final: back to LDS, where the updates below
+        // read their multipliers, and 16-lane row k stores column jb + k
+        // (rows jb .. jb+k+km) from there
+        const int r16 = lane & 15, d = (lane - c0) & 63;
+        if (lane < 16) {
+            unroll<NB>([&](auto k_) __attribute__((always_inline)) {
+                constexpr int k = decltype(k_)::value;
+                unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                    constexpr int m = decltype(m_)::value;
+                    pbuf[k * PS + 16 * m + r16] = T{px[k][m], py[k][m]};
+                });
+            });
+        }
+        WAVE_SYNC();
+        {
+            const int k = lane >> 4, j = jb + k;
+            const int last = min(k + kl, n - 1 - jb);
+            T *dst = ab + (size_t)min(j, n - 1) * ldab + KV - k;
+            unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                constexpr int m = decltype(m_)::value;
+                const R *x = reinterpret_cast<const R *>(pbuf + k * PS + 16 * m + r16);
+                const T v{x[0], x[1]};
+                if (j < n && 16 * m + r16 <= last) sz::gstore(dst + 16 * m + r16, v);
+            });
+            if (lane < NB && jb + lane < n) {
+                const int q4 = pick4(lane, jp[0], jp[1], jp[2], jp[3]);
+                *sz::gmem(ipiv + jb + lane) = jb + lane + q4 + 1;
+                if constexpr (UT) {
+                    T y;
+                    y.x = pick4(lane, yx[0], yx[1], yx[2], yx[3]);
+                    y.y = pick4(lane, yy[0], yy[1], yy[2], yy[3]);
+                    sz::gstore(bv + jb + lane, y);
+                }
+            }
+        }
+
+        // ---- 2. the four interchanges and updates on every column
+        unroll<NB>([&](auto uc_) __attribute__((always_inline)) {
+            constexpr int u = decltype(uc_)::value;
+            if (jp[u] != 0)
+                slot_swap<u, u / 4 * 4, u + kl>(ax, ay, u + jp[u],
+                                                __ballot(d >= u && d <= jus[u]));
+            const R ux = ax[u], uy = ay[u];
+            if constexpr (UT) {
+                const T v = sz::cfnms(T{bx, by}, T{ux, uy}, T{yx[u], yy[u]});
+                const bool in = jb + u < n && d > u && d - u <= KV;
+                bx = pick(in, v.x, bx);
+                by = pick(in, v.y, by);
+            }
+            if (nz >> u & 1) {
+                R lx[NM], ly[NM];
+                unroll<NM>([&](auto m_) __attribute__((always_inline)) {
+                    constexpr int m = decltype(m_)::value;
+                    const T v = pbuf[u * PS + 16 * m + r16];
+                    lx[m] = v.x;
+                    ly[m] = v.y;
+                });
+                panel_update<u + 1, u + kl>(ax, ay, lx, ly, ux, uy);
+                // Columns beyond ju have U(j, c) = 0, which a finite
+                // multiplier leaves alone but an infinite one or a NaN does
+                // not: no step has reached them, so they are read again.
+                if (odd >> u & 1) {
+                    const int c = jb + d;
+                    if (d > jus[u] && c < n) {
+                        const T *col = ab + (size_t)c * ldab + KV - d;
+                        unroll<PR>([&](auto s_) __attribute__((always_inline)) {
+                            constexpr int s = decltype(s_)::value;
+                            const T v = sz::gload(jb + s < n ? col + s : ab);
+                            const bool ok = d - s <= ku && jb + s < n;
+                            ax[s] = pick(ok, v.x, R(0));
+                            ay[s] = pick(ok, v.y, R(0));
+                        });
                     }
                 }
             }
-
-            // ---- rank-1 update of rows j+1 .. j+km, columns j+1 .. ju
-            if constexpr (!UT)
-                if (prio) __builtin_amdgcn_s_setprio(0);
-            if (nz && km > 0) {
-                if (d >= 1 && d <= ju - j) {
-#pragma unroll
-                    for (int s = 0; s < WR; ++s) {
-                        // multiplier of slot s from the lane of its row (a
-                        // scalar operand: no LDS traffic in the update)
-                        const int r = s - u < 0 ? s - u + WR : s - u;
-                        T m;
-                        m.x = readlane_r(lz.x, r);
-                        m.y = readlane_r(lz.y, r);
-                        a[s] = sz::cfnms(a[s], m, uc);
+            if constexpr (NT > 0) {
+                if (jus[u] >= 64 && (nz >> u & 1)) {       // a far pivot reached the tail
+                    if (lane < NT && 64 + lane <= jus[u] && jp[u] != 0) {
+                        R *x = reinterpret_cast<R *>(tail + lane * PR + u);
+                        R *y = reinterpret_cast<R *>(tail + lane * PR + u + jp[u]);
+                        const R x0 = x[0], x1 = x[1];
+                        x[0] = y[0];
+                        x[1] = y[1];
+                        y[0] = x0;
+                        y[1] = x1;
                     }
-                }
-                if constexpr (NTAIL > 0) {
-                    if (ju >= j + 64 && lane < NTAIL && j + 64 + lane <= ju) {
-                        int ts = th + lane;
-                        if (ts >= NTAIL) ts -= NTAIL;
-                        R *tc = reinterpret_cast<R *>(tail + ts * TW);
-                        const T ut{tc[2 * j0], tc[2 * j0 + 1]};
-                        for (int p = 0; p < WR; ++p) {
-                            int s = p - ob;                 // register slot of row p
-                            if (s < 0) s += WR;
-                            const T x = sz::cfnms(T{tc[2 * p], tc[2 * p + 1]}, lbuf[s], ut);
-                            tc[2 * p] = x.x;
-                            tc[2 * p + 1] = x.y;
-                            tc[2 * (p + WR)] = x.x;
-                            tc[2 * (p + WR) + 1] = x.y;
+                    WAVE_SYNC();
+                    const int t = lane >> 3;
+                    if (64 + t <= jus[u]) {
+                        const R *tu = reinterpret_cast<const R *>(tail + t * PR + u);
+                        const T ut{tu[0], tu[1]};
+                        for (int s = u + 1 + (lane & 7); s <= u + kl; s += 8) {
+                            R *x = reinterpret_cast<R *>(tail + t * PR + s);
+                            const R *lm = reinterpret_cast<const R *>(pbuf + u * PS + s);
+                            const T v = sz::cfnms(T{x[0], x[1]}, T{lm[0], lm[1]}, ut);
+                            x[0] = v.x;
+                            x[1] = v.y;
                         }
                     }
+                    WAVE_SYNC();
                 }
             }
-            WAVE_SYNC();
+        });
 
-            // ---- column j leaves: its lane takes column j+64 (the tail's
-            // first column, or zeros); row j leaves: slot u takes row j+WR
-            if (d == 0) {
-                if constexpr (NTAIL > 0) {
-                    const T *tc = tail + th * TW + ob;   // register order
-#pragma unroll
-                    for (int s = 0; s < WR; ++s) a[s] = tc[s];
-                    if constexpr (UT) breg = tailb[th];
-                } else {
-#pragma unroll
-                    for (int s = 0; s < WR; ++s) {
-                        a[s].x = R(0);
-                        a[s].y = R(0);
-                    }
-                    if constexpr (UT) breg = sel0(j + 64 < n, qb[u % WV_PF]);
-                }
-            }
-            {
-                const int dn = (lane - c0 - 1) & 63;   // offset from column j+1
-                const bool ok = j + WR < n && j + 1 + dn < n && dn <= KV;
-                const T e = qv[u % WV_PF];
-                a[u].x = ok ? e.x : R(0);
-                a[u].y = ok ? e.y : R(0);
-                if (replay && d >= 1 && d < WV_BS - u) tcol[u + d][u] = a[u];   // row j+WR
-                qv[u % WV_PF] = raw(j + WV_PF + WR,
-                                    j + WV_PF + 1 + ((lane - c0 - WV_PF - 1) & 63));
-            }
-            if constexpr (NTAIL > 0) {
-                WAVE_SYNC();
-                if (lane < WR) {
-                    tail[th * TW + lane] = T{R(0), R(0)};
-                    tail[th * TW + lane + WR] = T{R(0), R(0)};
-                }
-                WAVE_SYNC();
-                const int th1 = th + 1 == NTAIL ? 0 : th + 1;
-                if (lane < NTAIL) {
-                    int ts = th1 + lane;
-                    if (ts >= NTAIL) ts -= NTAIL;
-                    const bool ok = j + WR < n && j + 65 + lane < n;
-                    T e = qt[u % WV_PF];
-                    e.x = ok ? e.x : R(0);
-                    e.y = ok ? e.y : R(0);
-                    tail[ts * TW + j0] = e;
-                    tail[ts * TW + j0 + WR] = e;
-                }
-                qt[u % WV_PF] = raw(j + WV_PF + WR,
-                                    lane < NTAIL ? j + WV_PF + 65 + lane : n);
-                // the column entering the tail (j+kl+ku+1) brings its b
-                if constexpr (UT) {
-                    if (lane == 0) tailb[th] = sel0(j + KV + 1 < n, qb[u % WV_PF]);
-                }
-                th = th1;
-            }
-            if constexpr (UT)
-                qb[u % WV_PF] = sz::gload(bv + min(j + WV_PF + BNEW, n - 1));
-            WAVE_SYNC();
-            c0 = (c0 + 1) & 63;
+        asm volatile("" : "+v"(lane));
+        const bool leaving = ((lane - c0) & 63) < NB;    // a panel column's lane
+        // what the loads brought, before this block's stores join their queue
+        R qx[NB], qy[NB], qtx = R(0), qty = R(0), qbx = R(0), qby = R(0);
+        {
+            unroll<NB>([&](auto i_) __attribute__((always_inline)) {
+                constexpr int i = decltype(i_)::value;
+                take_lds(&qbuf[i * 64], lane, qx[i], qy[i]);
+            });
+            if constexpr (NT > 0) take_lds(&qbuf[NB * 64], lane, qtx, qty);
+            if constexpr (UT) take_lds(&qbuf[(NB + 1) * 64], lane, qbx, qby);
         }
-        // rename the slots: row jb+WV_BS+s moves to slot s
-        T t[WR];
-#pragma unroll
-        for (int s = 0; s < WR; ++s) t[s] = a[(s + WV_BS) % WR];
-#pragma unroll
-        for (int s = 0; s < WR; ++s) a[s] = t[s];
-        ob = ob + WV_BS >= WR ? ob + WV_BS - WR : ob + WV_BS;
+        __builtin_amdgcn_sched_barrier(0);
+
+        // ---- 3. U rows of the window's columns and of the tail's
+        const int row = lane & 3;
+        {
+            const int d = (lane - c0) & 63, c = jb + d;
+            if (!leaving && c < n) {
+                T *dst = ab + (size_t)c * ldab + KV - d;
+                unroll<NB>([&](auto i_) __attribute__((always_inline)) {
+                    constexpr int i = decltype(i_)::value;
+                    if (d - i <= KV) sz::gstore(dst + i, T{ax[i], ay[i]});
+                });
+            }
+            if constexpr (NT > 0) {
+                const int t = lane >> 2, ct = jb + 64 + t;
+                if (lane < NT * NB && ct < n && 64 + t - row <= KV) {
+                    const R *x = reinterpret_cast<const R *>(tail + t * PR + row);
+                    sz::gstore(ab + (size_t)ct * ldab + KV - 64 - t + row, T{x[0], x[1]});
+                }
+            }
+        }
+
+        // ---- the next block: slots renamed by NB, leaving lanes take the
+        // columns after the window's last, the next rows enter
+        // (as a loop this becomes a memmove, which keeps the arrays in scratch)
+        unroll<PR - NB>([&](auto s_) __attribute__((always_inline)) {
+            constexpr int s = decltype(s_)::value;
+            ax[s] = ax[s + NB];
+            ay[s] = ay[s + NB];
+        });
+        if constexpr (NT > 0) {
+            if constexpr (UT) {
+                T tb{R(0), R(0)};
+                if (lane < NT) {
+                    const R *x = reinterpret_cast<const R *>(tailb + lane);
+                    tb = T{x[0], x[1]};
+                    unroll<NB>([&](auto uc_) __attribute__((always_inline)) {
+                        constexpr int u = decltype(uc_)::value;
+                        const R *w = reinterpret_cast<const R *>(tail + lane * PR + u);
+                        if (jb + u < n && 64 + lane - u <= KV && jb + 64 + lane < n)
+                            tb = sz::cfnms(tb, T{w[0], w[1]}, T{yx[u], yy[u]});
+                    });
+                }
+                WAVE_SYNC();
+                if (lane < NT) tailb[lane] = tb;
+                WAVE_SYNC();
+                {
+                    const R *x = reinterpret_cast<const R *>(tailb + (leaving ? (lane - c0) & 63 : 0));
+                    bx = leaving ? x[0] : bx;
+                    by = leaving ? x[1] : by;
+                }
+                const bool in = jb + NB + 64 + lane < n;
+                const R *up = reinterpret_cast<const R *>(tailb + (lane < NB ? lane + NB : 0));
+                const R nbx = lane < NB ? up[0] : in ? qbx : R(0);
+                const R nby = lane < NB ? up[1] : in ? qby : R(0);
+                WAVE_SYNC();
+                if (lane < NT) tailb[lane] = T{nbx, nby};
+            }
+            if (leaving) {
+                // (keeps the branch, whose reads land in place: speculated,
+                // they would take a select each)
+                asm volatile("; leaving");
+                const T *col = tail + ((lane - c0) & 63) * PR + NB;
+                unroll<PR - NB>([&](auto s_) __attribute__((always_inline)) {
+                    constexpr int s = decltype(s_)::value;
+                    const R *x = reinterpret_cast<const R *>(col + s);
+                    ax[s] = x[0];
+                    ay[s] = x[1];
+                });
+            }
+            // the tail's later columns move up, its last four are new
+            constexpr int MV = (NT - NB) * (PR - NB), MI = (MV + 63) / 64;
+            R mvx[MI], mvy[MI];
+            unroll<MI>([&](auto e_) __attribute__((always_inline)) {
+                constexpr int e = decltype(e_)::value;
+                const int x = min(lane + 64 * e, MV - 1), t = x / (PR - NB);
+                const T v = tail[(t + NB) * PR + NB + x - t * (PR - NB)];
+                mvx[e] = v.x;
+                mvy[e] = v.y;
+            });
+            WAVE_SYNC();
+            unroll<MI>([&](auto e_) __attribute__((always_inline)) {
+                constexpr int e = decltype(e_)::value;
+                const int x = lane + 64 * e, t = x / (PR - NB);
+                if (x < MV) {
+                    tail[t * PR + x - t * (PR - NB)] = T{mvx[e], mvy[e]};
+                    R z = R(0);          // (a zero held through the loop gets spilled)
+                    asm volatile("" : "+v"(z));
+                    tail[(t + NB) * PR + x - t * (PR - NB)] = T{z, z};
+                }
+            });
+            if (lane < NT * NB) {
+                const int t = lane >> 2;
+                const bool ok = jb + NB + 64 + t < n && jb + PR + row < n && t <= KV - 64 + row;
+                tail[t * PR + PR - NB + row] = T{ok ? qtx : R(0), ok ? qty : R(0)};
+            }
+        } else {
+            if (leaving) {
+                asm volatile("; leaving");
+                unroll<PR - NB>([&](auto s_) __attribute__((always_inline)) {
+                    constexpr int s = decltype(s_)::value;
+                    ax[s] = ay[s] = R(0);
+                });
+                if constexpr (UT) {
+                    const bool in = jb + 64 + ((lane - c0) & 63) < n;
+                    bx = in ? qbx : R(0);
+                    by = in ? qby : R(0);
+                }
+            }
+        }
+        unroll<NB>([&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value;
+            const int dn = (lane - c0 - NB) & 63;
+            const bool ok = jb + NB + dn < n && jb + PR + i < n && dn >= i && dn <= KV + i;
+            ax[PR - NB + i] = pick(ok, qx[i], R(0));
+            ay[PR - NB + i] = pick(ok, qy[i], R(0));
+        });
+        WAVE_SYNC();
     }
     if (lane == 0 && info) *sz::gmem(info + sys) = first_zero;
 }
 
-// 1 when a batch of one-wave factorizations leaves some SIMDs with two waves
-// and most with one (between one and two systems per SIMD): 1152 systems
-// take 1.69 ms instead of 1.82 with the pivot chain prioritised; at two or
-// more waves per SIMD it costs 1%.
-int wave_priority(int nsys)
+// Launches k_gbtrf_panel for the band shapes it is instantiated for -- kl =
+// ku = 34 (five interleaved fields, k = 8 operators), kl = ku = 24 (k = 6)
+// and kl = 34, ku = 20 -- and returns whether the shape is one of them.
+template <typename R, bool UT>
+bool launch_panel(int n, int kl, int ku, void *ab, int ldab, long long sab, int *ipiv,
+                  long long sipiv, int *info, const int *skip, int nsys, void *b,
+                  long long sb, const sz::gsys *gs, hipStream_t stream)
 {
-    static const int simds = [] {
-        int dev = 0, cus = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-                hipSuccess)
-            return 0;
-        return 4 * cus;
-    }();
-    return nsys > simds && nsys < 2 * simds ? 1 : 0;
+#define SZ_PANEL(WR_, KV_)                                                      \
+    hipLaunchKernelGGL((k_gbtrf_panel<R, WR_, KV_, UT, panel_waves(sizeof(R), WR_, UT)>), \
+                       dim3(nsys), dim3(64), 0, stream, n,                      \
+                       reinterpret_cast<cpx<R> *>(ab), ldab, sab, ipiv, sipiv, info, \
+                       skip, nsys, reinterpret_cast<cpx<R> *>(b), sb, gs)
+    if (kl == 34 && ku == 34) SZ_PANEL(35, 68);
+    else if (kl == 24 && ku == 24) SZ_PANEL(25, 48);
+    else if (kl == 34 && ku == 20) SZ_PANEL(35, 54);
+    else return false;
+#undef SZ_PANEL
+    return true;
 }
 
-// Factorization kernels: k_gbtrf_wave (one wavefront per system, window in
-// registers) for the band shapes it is instantiated for -- kl = ku = 34
-// (five interleaved fields, k = 8 operators), kl = ku = 24 (k = 6) and
-// kl = 34, ku = 20 -- and the LDS window kernel k_gbtrf for every other
-// shape.  SZ_GBTRF_KERNEL: "lds" (or "lds64"/"lds128", fewer threads) forces
-// the LDS kernel; "v4"/"v2" run the wave kernel in shorter unrolled blocks.
+// Factorization kernels: k_gbtrf_panel for the channel band shapes and the
+// LDS window kernel k_gbtrf for every other shape.  SZ_GBTRF_KERNEL = "lds"
+// (or "lds64"/"lds128", fewer threads) forces the LDS kernel.
 template <typename R>
 int launch_gbtrf(int n, int kl, int ku, void *ab, int ldab, long long sab,
                  int *ipiv, long long sipiv, int *info, const int *skip,
@@ -1328,29 +1672,10 @@ int launch_gbtrf(int n, int kl, int ku, void *ab, int ldab, long long sab,
     if (nsys < 0) return -10;
     if (nsys == 0 || n == 0) return 0;
     static const char *sel = getenv("SZ_GBTRF_KERNEL");
-    if (!(sel && sel[0] == 'l')) {
-        const int bs = (sel && sel[0] == 'v' && sel[1] == '2') ? 2
-                     : (sel && sel[0] == 'v' && sel[1] == '4') ? 4 : 8;
-        bool done = true;
-#define SZ_WAVE(WR_, KV_, BS_)                                                  \
-        hipLaunchKernelGGL((k_gbtrf_wave<R, WR_, KV_, BS_>), dim3(nsys), dim3(64), 0, \
-                           stream, n, reinterpret_cast<cpx<R> *>(ab), ldab, sab, ipiv, \
-                           sipiv, info, skip, nsys, nullptr, 0, prio)
-        const int prio = wave_priority(nsys);
-        if (kl == 34 && ku == 34) {
-            if (bs == 2) SZ_WAVE(35, 68, 2);
-            else if (bs == 4) SZ_WAVE(35, 68, 4);
-            else SZ_WAVE(35, 68, 8);
-        } else if (kl == 24 && ku == 24) {
-            SZ_WAVE(25, 48, 8);
-        } else if (kl == 34 && ku == 20) {
-            SZ_WAVE(35, 54, 8);
-        } else {
-            done = false;
-        }
-#undef SZ_WAVE
-        if (done) return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
-    }
+    if (!(sel && sel[0] == 'l') &&
+        launch_panel<R, false>(n, kl, ku, ab, ldab, sab, ipiv, sipiv, info, skip, nsys,
+                               nullptr, 0, nullptr, stream))
+        return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
     const size_t lds = ((size_t)(kl + 1) * (kl + ku + 1) + (kl + ku + 1) + (kl + 1))
                        * sizeof(cpx<R>);
     if (lds > LDS_MAX) return SZ_ERR_LDS;
@@ -1393,18 +1718,9 @@ int launch_gbtrf_ut(int n, int kl, int ku, void *ab, int ldab, long long sab,
     if (nsys == 0 || n == 0) return 0;
     static const char *sel = getenv("SZ_GBTRF_KERNEL");
     if (sel && sel[0] == 'l') return 1;
-    // 4-step blocks: with the U^T solve and the block-column transposes the
-    // 8-step loop body outgrows the instruction cache (110 KB of code);
-    // 4 steps (5.41 ms per 4560 systems) beat 8 (5.60) and equal 6
-#define SZ_WAVE_UT(WR_, KV_)                                                    \
-    hipLaunchKernelGGL((k_gbtrf_wave<R, WR_, KV_, 4, true>), dim3(nsys), dim3(64), 0, \
-                       stream, n, reinterpret_cast<cpx<R> *>(ab), ldab, sab, ipiv, \
-                       sipiv, info, nullptr, nsys, reinterpret_cast<cpx<R> *>(b), sb)
-    if (kl == 34 && ku == 34) SZ_WAVE_UT(35, 68);
-    else if (kl == 24 && ku == 24) SZ_WAVE_UT(25, 48);
-    else if (kl == 34 && ku == 20) SZ_WAVE_UT(35, 54);
-    else return 1;
-#undef SZ_WAVE_UT
+    if (!launch_panel<R, true>(n, kl, ku, ab, ldab, sab, ipiv, sipiv, info, nullptr, nsys,
+                               b, sb, nullptr, stream))
+        return 1;
     return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
 }
 
@@ -1539,31 +1855,18 @@ int launch_gbtrs(char trans, int n, int kl, int ku, int nrhs, const void *ab,
 
 // Grouped launches: every system of gs (orders up to nmax, band storage at
 // gs[s].ab with leading dimension ldab = 2 kl + ku + 1) in one launch.
-// The wave factorization kernel takes the channel band shapes (kl = ku = 34
-// and 24); bs selects its unrolled block (4 or 8 steps).
+// The panel kernel takes the channel band shapes; no other is grouped.
 template <typename R>
 int launch_gbtrf_grouped(int kl, int ku, void *ab, int ldab, int *ipiv, int *info,
-                         const int *skip, const sz::gsys *gs, int nsys, int bs,
+                         const int *skip, const sz::gsys *gs, int nsys,
                          hipStream_t stream)
 {
     if (nsys <= 0) return nsys < 0 ? -10 : 0;
     if (ldab != 2 * kl + ku + 1) return -5;
-    const int prio = 0;
-    cpx<R> *a = reinterpret_cast<cpx<R> *>(ab);
-#define SZ_WAVE_G(WR_, KV_, BS_)                                                 \
-    hipLaunchKernelGGL((k_gbtrf_wave<R, WR_, KV_, BS_>), dim3(nsys), dim3(64), 0,  \
-                       stream, 0, a, ldab, 0LL, ipiv, 0LL, info, skip, nsys,     \
-                       nullptr, 0LL, prio, gs)
-    if (kl == 34 && ku == 34) {
-        if (bs == 4) SZ_WAVE_G(35, 68, 4);
-        else SZ_WAVE_G(35, 68, 8);
-    } else if (kl == 24 && ku == 24) {
-        if (bs == 4) SZ_WAVE_G(25, 48, 4);
-        else SZ_WAVE_G(25, 48, 8);
-    } else {
+    if (!((kl == 34 && ku == 34) || (kl == 24 && ku == 24))) return SZ_ERR_LDS;
+    if (!launch_panel<R, false>(0, kl, ku, ab, ldab, 0, ipiv, 0, info, skip, nsys, nullptr,
+                                0, gs, stream))
         return SZ_ERR_LDS;
-    }
-#undef SZ_WAVE_G
     return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
 }
 
@@ -1642,14 +1945,14 @@ extern "C" {
 
 int sz_internal_gbtrf_grouped(int single, int kl, int ku, void *ab, int ldab,
                               int *ipiv, int *info, const int *skip,
-                              const void *gs, int nsys, int bs, void *stream)
+                              const void *gs, int nsys, void *stream)
 {
     const sz::gsys *g = static_cast<const sz::gsys *>(gs);
     if (single)
         return launch_gbtrf_grouped<float>(kl, ku, ab, ldab, ipiv, info, skip, g,
-                                           nsys, bs, (hipStream_t)stream);
+                                           nsys, (hipStream_t)stream);
     return launch_gbtrf_grouped<double>(kl, ku, ab, ldab, ipiv, info, skip, g, nsys,
-                                        bs, (hipStream_t)stream);
+                                        (hipStream_t)stream);
 }
 
 // 1 when the single precision grouped transposed solve of this band shape

@@ -47,7 +47,7 @@ extern "C" int sz_internal_band_split_grouped(int kl, int ku, const void *gs, in
 extern "C" int sz_internal_gbtrf_grouped(int single, int kl, int ku, void *ab,
                                          int ldab, int *ipiv, int *info,
                                          const int *skip, const void *gs,
-                                         int nsys, int bs, void *stream);
+                                         int nsys, void *stream);
 extern "C" int sz_internal_gbtrs_grouped(int single, char trans, int kl, int ku,
                                          const void *ab, int ldab,
                                          const int *ipiv, void *b,
@@ -817,11 +817,6 @@ int sz_prec_sys0(const sz_prec *h, int k)
     return -1;
 }
 
-void sz_prec_set_lu_bs(sz_prec *h, int bs)
-{
-    if (h) h->p.lu_bs = bs;
-}
-
 void sz_prec_set_graph(sz_prec *h, int graph)
 {
     if (h) h->p.graph = graph ? 1 : 0;
@@ -965,7 +960,7 @@ int single_pass(sz_prec *h, sz_prec::slot &sl, int slot, const p_args &A0, int p
     for (const auto &c : h->classes) {
         rc = sz_internal_gbtrf_grouped(1, c.KL, c.KU, nullptr, c.ldlu, nullptr,
                                        h->finfo + c.s0, h->fskip + c.s0,
-                                       c.gs[(size_t)slot], c.ns, h->p.lu_bs, st);
+                                       c.gs[(size_t)slot], c.ns, st);
         if (rc) return rc;
         if (c.split) {
             rc = sz_internal_band_split_grouped(

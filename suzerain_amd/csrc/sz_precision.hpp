@@ -95,7 +95,6 @@ struct sz_prec_params {
     int reuse;            // keep factors between calls (apprx semantics)
     int graph;            // no host waits: restart pass always enqueued,
                           // no double fallback (capturable in a hipGraph)
-    int lu_bs;            // factorization unroll (4 or 8; 0 = default)
 };
 
 // One member's operator and right hand side for one call: the imexop
@@ -153,5 +152,4 @@ void sz_prec_counts(const sz_prec *h, int *factored, int *restarted,
 // Total systems over all members.
 int sz_prec_nsys(const sz_prec *h);
 // Factorization unroll (autotuner) and graph mode switches.
-void sz_prec_set_lu_bs(sz_prec *h, int bs);
 void sz_prec_set_graph(sz_prec *h, int graph);

@@ -1,0 +1,90 @@
+"""The panel factorization (four columns at a time) of the channel band shapes
+where it can go wrong: orders around its block of four columns, its 64-column
+window and its last rows; pivots far enough to reach the columns beyond the
+window; zero pivots; and infinities, whose updates must leave the columns no
+interchange has reached as they are.  Compared with the oracle bit for bit
+(a NaN equals a NaN), as LAPACK's column-by-column loop orders the sums.
+"""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(34, 34), (24, 24), (34, 20)]
+
+
+def _bands(rng, nb, N, kl, ku, dom):
+    ldab = 2 * kl + ku + 1
+    ab = np.zeros((nb, N, ldab), dtype=np.complex128)
+    for j in range(N):
+        lo, hi = max(0, j - ku), min(N, j + kl + 1)
+        r = kl + ku + np.arange(lo, hi) - j
+        ab[:, j, r] = (rng.standard_normal((nb, hi - lo)) +
+                       1j * rng.standard_normal((nb, hi - lo)))
+    ab[:, :, kl + ku] += dom
+    return ab
+
+
+def _check(gpu, ab, kl, ku, precision):
+    import torch
+    import suzerain_amd as sa
+    if precision == "c":
+        ab = ab.astype(np.complex64)
+    N, ldab = ab.shape[1:]
+    abd = torch.from_numpy(ab).to(gpu)
+    ipiv, info = sa.gbtrf(abd, kl, ku, precision=precision)
+    lu, ipiv, info = abd.cpu().numpy(), ipiv.cpu().numpy(), info.cpu().numpy()
+    for s in range(ab.shape[0]):
+        ref = ab[s].reshape(-1).copy()
+        with np.errstate(all="ignore"):
+            rinfo, rpiv = oracle.zgbtrf(N, kl, ku, ref, ldab)
+        assert info[s] == rinfo
+        np.testing.assert_array_equal(ipiv[s], rpiv)
+        np.testing.assert_array_equal(lu[s], ref.reshape(N, ldab))
+    return ipiv
+
+
+@pytest.mark.parametrize("precision", ["z", "c"])
+@pytest.mark.parametrize("kl,ku", SHAPES)
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 35, 37, 63, 64, 65, 68, 69, 70, 71,
+                               72, 73, 76, 103, 135])
+def test_orders_around_the_blocks(gpu, N, kl, ku, precision):
+    rng = np.random.default_rng(1000 * kl + ku + N)
+    _check(gpu, _bands(rng, 3, N, kl, ku, 0.0), kl, ku, precision)
+    _check(gpu, _bands(rng, 2, N, kl, ku, 20.0), kl, ku, precision)
+
+
+@pytest.mark.parametrize("precision", ["z", "c"])
+@pytest.mark.parametrize("kl,ku", SHAPES)
+def test_far_pivots_and_ties(gpu, kl, ku, precision):
+    """The last sub-diagonal dominates (every pivot kl rows away, so every
+    fill-in column is used), then entries of equal magnitude (the first wins)
+    and magnitudes that differ in the low word only."""
+    rng = np.random.default_rng(kl + ku)
+    N = 150
+    ab = _bands(rng, 3, N, kl, ku, 0.0)
+    ab[0, :, 2 * kl + ku] *= 50.0
+    ab[1] = np.where(ab[1] != 0, np.sign(ab[1].real), 0)
+    ab[2] = np.where(ab[2] != 0, 1 + 1e-12 * ab[2].real, 0)
+    for j in range(N):                       # entries past the last row stay zero
+        ab[:, j, kl + ku + N - j:] = 0
+    piv = _check(gpu, ab, kl, ku, precision)
+    assert (piv[0] - np.arange(1, N + 1)).max() == kl
+
+
+@pytest.mark.parametrize("kl,ku", SHAPES)
+def test_infinities_and_zero_columns(gpu, kl, ku):
+    """An infinite entry, a NaN off the diagonal, a NaN in a pivot row and a
+    column of zeros, each in a system of its own."""
+    rng = np.random.default_rng(7 * kl + ku)
+    N = 120
+    ab = _bands(rng, 5, N, kl, ku, 20.0)
+    ab[0, 50, kl + ku + 2] = np.inf
+    ab[1, 41, kl + ku + 5] = np.nan
+    ab[2, 62, kl + ku] = complex(np.nan, 1.0)
+    ab[3, 33, :] = 0.0
+    ab[4, 70, kl + ku] = 5e-324              # 1/pivot overflows
+    ab[4, 70, kl + ku + 1:] = 0.0
+    _check(gpu, ab, kl, ku, "z")
