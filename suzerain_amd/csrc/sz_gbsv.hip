@@ -32,6 +32,7 @@
 // the compiler's DPP move for 64-bit values (its builtin takes 32 bits only)
 __device__ double sz_update_dpp(double, double, int, int, int, bool)
     __asm("llvm.amdgcn.update.dpp.f64");
+__device__ int sz_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 
 namespace {
 
@@ -64,15 +65,15 @@ __device__ __forceinline__ R dpp_r(R v)
 {
     if constexpr (sizeof(R) == 8) {
         const long long b = __builtin_bit_cast(long long, v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, true);
         const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF,
-                                                   0xF, false);
+                                                   0xF, true);
         return __builtin_bit_cast(R, (long long)(((unsigned long long)(unsigned)hi << 32)
                                                  | (unsigned)lo));
     } else {
         return __builtin_bit_cast(
             R, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF,
-                                           0xF, false));
+                                           0xF, true));
     }
 }
 
@@ -350,17 +351,91 @@ __device__ inline cpx<R> cj_if(cpx<R> v, bool c)
     return r;
 }
 
+template <int... I, typename F>
+__device__ __forceinline__ void unroll_impl(F &&f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int K, typename F>
+__device__ __forceinline__ void unroll(F &&f)
+{
+    unroll_impl(f, std::make_integer_sequence<int, K>{});
+}
+
+// L^T x = y and the interchanges, the second half of a transposed solve, on x
+// in LDS by one wavefront.
+template <typename R>
+__device__ __forceinline__ void lt_sweep(int n, int kl, int kv,
+                                         const cpx<R> *__restrict__ ab, int ldab,
+                                         const int *__restrict__ ipiv, bool cj, cpx<R> *x,
+                                         int tid)
+{
+    using T = cpx<R>;
+    // L^T x = y then undo the interchanges, descending.  Lane r
+    // forms the terms r, r+64, ... of the dot product with the
+    // multipliers of column j (one contiguous run, prefetched a few
+    // steps ahead) and the butterfly combines them.
+    if (kl > 0 && n > 1) {
+        constexpr int QP = 4;
+        auto laddr = [&](int jj, int r) -> size_t {   // L(jj+1+r, jj)
+            const bool ok = jj >= 0 && r < min(kl, n - 1 - jj);
+            return ok ? (size_t)jj * ldab + kv + 1 + r : 0;
+        };
+        T l1[QP], l2[QP];
+        int qp[QP];
+#pragma unroll
+        for (int u = 0; u < QP; ++u) {
+            l1[u] = ab[laddr(n - 2 - u, tid)];
+            l2[u] = ab[laddr(n - 2 - u, tid + TRS_NT)];
+            qp[u] = ipiv[max(n - 2 - u, 0)];
+        }
+        for (int jb = n - 2; jb >= 0; jb -= QP) {
+#pragma unroll
+            for (int u = 0; u < QP; ++u) {
+                const int j = jb - u;
+                if (j < 0) break;
+                const int lm = min(kl, n - 1 - j);
+                T acc = {0, 0};
+                if (tid < lm) acc = sz::cfma(acc, cj_if(l1[u], cj), x[j + 1 + tid]);
+                if (tid + TRS_NT < lm)
+                    acc = sz::cfma(acc, cj_if(l2[u], cj), x[j + 1 + tid + TRS_NT]);
+                for (int r = tid + 2 * TRS_NT; r < lm; r += TRS_NT)
+                    acc = sz::cfma(acc, cj_if(ab[laddr(j, r)], cj), x[j + 1 + r]);
+                acc = wave_csum(acc);
+                if (tid == 0) {
+                    // component-wise (a struct copy here goes through
+                    // scratch)
+                    const T xo = x[j];
+                    const R xjx = xo.x - acc.x, xjy = xo.y - acc.y;
+                    int l = qp[u] - 1;
+                    if (l < j || l >= n) l = j;
+                    const R xlx = x[l].x, xly = x[l].y;
+                    x[l].x = xjx;
+                    x[l].y = xjy;
+                    if (l != j) {
+                        x[j].x = xlx;
+                        x[j].y = xly;
+                    }
+                }
+                l1[u] = ab[laddr(j - QP, tid)];
+                l2[u] = ab[laddr(j - QP, tid + TRS_NT)];
+                qp[u] = ipiv[max(j - QP, 0)];
+                LDS_BARRIER();
+            }
+        }
+    }
+}
+
 // trans: 0 = 'N', 1 = 'T', 2 = 'C'.  One 64-lane workgroup per system; the
 // right-hand side lives in LDS, one barrier per elimination step.
-// TR: transposed ('T'/'C'); LT_ONLY: only the L^T half (U^T already done
-// by the fused factorization), compiled without the U^T prefetch queues.
-template <typename R, bool TR, bool LT_ONLY = false>
+// TR: transposed ('T'/'C').
+template <typename R, bool TR>
 __global__ __launch_bounds__(TRS_NT)
 void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
              const cpx<R> *__restrict__ ab, int ldab, long long sab,
              const int *__restrict__ ipiv, long long sipiv,
              cpx<R> *__restrict__ b, int ldb, long long sb,
-             const int *__restrict__ skip, int nsys, int skip_ut,
+             const int *__restrict__ skip, int nsys,
              const sz::gsys *__restrict__ gs = nullptr)
 {
     using T = cpx<R>;
@@ -454,8 +529,7 @@ void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
             // x[k] receives U(k-t, k) y_{k-t} for t = kv .. 1, the order of
             // the sequential LAPACK loop, and no step needs a reduction.
             // Lane 0 keeps x[j+1] (its own update) for the next division.
-            // skip_ut: b already holds y (solved during the factorization).
-            if (!LT_ONLY && !skip_ut) {
+            {
                 constexpr int QP = 4;                  // steps prefetched ahead
                 const int t1 = tid + 1, t2 = tid + 1 + TRS_NT;
                 auto uaddr = [&](int jj, int t) -> size_t {   // U(jj, jj+t)
@@ -497,59 +571,7 @@ void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
                     }
                 }
             }
-            // L^T x = y then undo the interchanges, descending.  Lane r
-            // forms the terms r, r+64, ... of the dot product with the
-            // multipliers of column j (one contiguous run, prefetched a few
-            // steps ahead) and the butterfly combines them.
-            if (kl > 0 && n > 1) {
-                constexpr int QP = 4;
-                auto laddr = [&](int jj, int r) -> size_t {   // L(jj+1+r, jj)
-                    const bool ok = jj >= 0 && r < min(kl, n - 1 - jj);
-                    return ok ? (size_t)jj * ldab + kv + 1 + r : 0;
-                };
-                T l1[QP], l2[QP];
-                int qp[QP];
-#pragma unroll
-                for (int u = 0; u < QP; ++u) {
-                    l1[u] = ab[laddr(n - 2 - u, tid)];
-                    l2[u] = ab[laddr(n - 2 - u, tid + TRS_NT)];
-                    qp[u] = ipiv[max(n - 2 - u, 0)];
-                }
-                for (int jb = n - 2; jb >= 0; jb -= QP) {
-#pragma unroll
-                    for (int u = 0; u < QP; ++u) {
-                        const int j = jb - u;
-                        if (j < 0) break;
-                        const int lm = min(kl, n - 1 - j);
-                        T acc = {0, 0};
-                        if (tid < lm) acc = sz::cfma(acc, cj_if(l1[u], cj), x[j + 1 + tid]);
-                        if (tid + TRS_NT < lm)
-                            acc = sz::cfma(acc, cj_if(l2[u], cj), x[j + 1 + tid + TRS_NT]);
-                        for (int r = tid + 2 * TRS_NT; r < lm; r += TRS_NT)
-                            acc = sz::cfma(acc, cj_if(ab[laddr(j, r)], cj), x[j + 1 + r]);
-                        acc = wave_csum(acc);
-                        if (tid == 0) {
-                            // component-wise (a struct copy here goes through
-                            // scratch)
-                            const T xo = x[j];
-                            const R xjx = xo.x - acc.x, xjy = xo.y - acc.y;
-                            int l = qp[u] - 1;
-                            if (l < j || l >= n) l = j;
-                            const R xlx = x[l].x, xly = x[l].y;
-                            x[l].x = xjx;
-                            x[l].y = xjy;
-                            if (l != j) {
-                                x[j].x = xlx;
-                                x[j].y = xly;
-                            }
-                        }
-                        l1[u] = ab[laddr(j - QP, tid)];
-                        l2[u] = ab[laddr(j - QP, tid + TRS_NT)];
-                        qp[u] = ipiv[max(j - QP, 0)];
-                        LDS_BARRIER();
-                    }
-                }
-            }
+            lt_sweep(n, kl, kv, ab, ldab, ipiv, cj, x, tid);
         }
         for (int i = tid; i < n; i += TRS_NT) bs[i] = x[i];
         LDS_BARRIER();
@@ -563,6 +585,495 @@ void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
         __builtin_amdgcn_wave_barrier();                                      \
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");                \
     } while (0)
+
+// ------------------------------------------------------- register solve
+// The solves of k_gbtrs with the active part of the right hand side in
+// registers, for the bands launch_gbtrs_reg admits: one wavefront per system,
+// row i in lane i mod 64, NR registers deep.  A finished row's lane takes the
+// row 64 NR further on from a prefetched register, so no value moves between
+// lanes: a step broadcasts one element by readlane and every lane updates its
+// own row, with the multiply-adds in the order of the LAPACK loops
+// (bit-identical).
+//   * SOLVE_N: L forward (multipliers of column j, interchanges by readlane and
+//     writelane), then U backward (column j above the diagonal);
+//   * SOLVE_T: U^T forward: lane = column, four rows of U (64 contiguous bytes
+//     of the column) per load; then L^T backward, whose dot products are summed
+//     as k_gbtrs sums them, by distance from the diagonal: there the window
+//     itself moves by one lane a step;
+//   * SOLVE_LT: the L^T half alone, after a factorization that solved U^T.
+// The columns of the next PF steps are in flight: the barrier to the scheduler
+// before each fetch keeps a load behind the last use of the registers it fills
+// (else they are copied, and the copy waits for the load).
+// Bound by instruction issue of one wavefront (75 instructions a step; the
+// division by U(j, j) has its reciprocal formed 64 at a time), for thousands of
+// systems by issue of the SIMD; the factors' bytes take a third of the time.
+// Measured, against x in LDS with a barrier a step: N of 576 systems n = 480,
+// kl = ku = 34: 459 -> 294 us (455 MB); T of 600 systems n = 301, kl 17, ku 11,
+// two right hand sides: 615 -> 253 us; L^T of 1520 systems n = 480, kl = 34:
+// 483 -> 334 us; N in float, 300 systems n = 200, kl = ku = 24: 37 -> 19 us.
+template <typename R>
+__device__ __forceinline__ R sel(bool c, R a, R b) { return c ? a : b; }
+
+// v moved up by one lane, lane 0 taking first
+template <typename R>
+__device__ __forceinline__ R wave_shr(R v, R first)
+{
+    if constexpr (sizeof(R) == 8) {
+        const long long b = __builtin_bit_cast(long long, v);
+        const long long f = __builtin_bit_cast(long long, first);
+        const int lo = __builtin_amdgcn_update_dpp((int)f, (int)b, 0x138, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp((int)(f >> 32), (int)(b >> 32), 0x138, 0xf,
+                                                   0xf, false);
+        return __builtin_bit_cast(R, (long long)(((unsigned long long)(unsigned)hi << 32)
+                                                 | (unsigned)lo));
+    } else {
+        return __builtin_bit_cast(R, __builtin_amdgcn_update_dpp(
+            __builtin_bit_cast(int, first), __builtin_bit_cast(int, v), 0x138, 0xf, 0xf,
+            false));
+    }
+}
+
+// a + b over the two rows of 16 lanes (16) or halves of the wave (32) that the
+// gfx950 swaps exchange: [r0 + r1, r0 + r1, r2 + r3, r2 + r3] for 16
+template <int W, typename R>
+__device__ __forceinline__ R swap_add(R v)
+{
+    auto swap = [](unsigned a) __attribute__((always_inline)) {
+        if constexpr (W == 16) return __builtin_amdgcn_permlane16_swap(a, a, false, false);
+        else return __builtin_amdgcn_permlane32_swap(a, a, false, false);
+    };
+    if constexpr (sizeof(R) == 8) {
+        const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+        const auto lo = swap((unsigned)b), hi = swap((unsigned)(b >> 32));
+        return __builtin_bit_cast(R, (unsigned long long)hi[0] << 32 | lo[0]) +
+               __builtin_bit_cast(R, (unsigned long long)hi[1] << 32 | lo[1]);
+    } else {
+        const auto w = swap(__builtin_bit_cast(unsigned, v));
+        return __builtin_bit_cast(R, (unsigned)w[0]) + __builtin_bit_cast(R, (unsigned)w[1]);
+    }
+}
+
+// wave_csum's sums, re valid in lane 0 and im in lane 1: the first exchange
+// sends one component and keeps the other, so the rest adds both at once.  An
+// addend's order within a sum never matters, its grouping stays the butterfly's.
+template <typename R>
+__device__ __forceinline__ R wave_csum01(R re, R im, bool odd)
+{
+    R v = sel(odd, im, re) + dpp_r<0xB1>(sel(odd, re, im));   // l ^ 1
+    v += dpp_r<0x4E>(v);                                      // l ^ 2
+    v += dpp_r<0x104>(v);                                     // row_shl:4
+    v += dpp_r<0x108>(v);                                     // row_shl:8
+    return swap_add<32>(swap_add<16>(v));
+}
+
+// v's 32-bit words of lane l replaced by w's (both uniform)
+template <typename R>
+__device__ __forceinline__ R writelane_r(R v, R w, int l)
+{
+    if constexpr (sizeof(R) == 8) {
+        const long long b = __builtin_bit_cast(long long, v);
+        const long long f = __builtin_bit_cast(long long, w);
+        const int lo = sz_writelane((int)f, l, (int)b);
+        const int hi = sz_writelane((int)(f >> 32), l, (int)(b >> 32));
+        return __builtin_bit_cast(R, (long long)(((unsigned long long)(unsigned)hi << 32)
+                                                 | (unsigned)lo));
+    } else {
+        return __builtin_bit_cast(R, sz_writelane(
+            __builtin_bit_cast(int, w), l, __builtin_bit_cast(int, v)));
+    }
+}
+
+// Division by a diagonal, one a lane.  Smith's quotient is
+// (x c1 + y c2, y c1 - x c2) / den with (c1, c2) = (1, ratio) or (ratio, 1).
+// With rec = 1 / den rounded, q = n rec corrected twice by fma(n - q den, rec)
+// is the rounded n / den (Markstein: the first correction leaves a neighbour
+// of n / den, the second starts from an exact remainder), as long as nothing
+// leaves the normal range: mid() keeps |n| and |den| far inside it, and any
+// other value, zero included, takes the division itself.
+template <typename R>
+struct smith {
+    R c1, c2, den, rec;
+    unsigned long long mid;
+};
+template <typename R>
+__device__ __forceinline__ bool mid(R a, R b)        // both of ordinary size
+{
+    constexpr int E = sizeof(R) == 8 ? 400 : 50;     // 2^-E <= |.| < 2^E
+    constexpr int SH = sizeof(R) == 8 ? 21 : 24;     // exponent, sign shifted out
+    constexpr unsigned BIAS = sizeof(R) == 8 ? 1023 : 127;
+    auto key = [](R v) __attribute__((always_inline)) {
+        unsigned h;
+        if constexpr (sizeof(R) == 8)
+            h = (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32);
+        else
+            h = __builtin_bit_cast(unsigned, v);
+        return (h << 1) - ((BIAS - E) << SH);
+    };
+    return max(key(a), key(b)) < (2u * E << SH);
+}
+template <typename R>
+__device__ __forceinline__ smith<R> smith_of(R zx, R zy)
+{
+    smith<R> d;
+    const bool big = fabs(zx) >= fabs(zy);
+    const R P = sel(big, zx, zy), Q = sel(big, zy, zx);
+    const R ratio = Q / P;
+    d.den = P + Q * ratio;
+    d.rec = R(1) / d.den;
+    d.c1 = sel(big, R(1), ratio);
+    d.c2 = sel(big, ratio, R(1));
+    d.mid = __ballot(mid(d.den, d.den));
+    return d;
+}
+
+// x / z in lane jj (returned in q there) and its value v, uniform
+template <typename R>
+__device__ __forceinline__ void smith_div(const smith<R> &d, int jj, R x, R y, R &qx, R &qy,
+                                          cpx<R> &v, bool &nz)
+{
+    const R n2 = x * d.c1 + y * d.c2, n3 = y * d.c1 - x * d.c2;
+    R a = n2 * d.rec, b = n3 * d.rec;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        a = __builtin_fma(__builtin_fma(-d.den, a, n2), d.rec, a);
+        b = __builtin_fma(__builtin_fma(-d.den, b, n3), d.rec, b);
+    }
+    nz = true;
+    if (!((__ballot(mid(n2, n3)) & d.mid) >> jj & 1)) {
+        nz = __ballot(sz::cnonzero(cpx<R>{x, y})) >> jj & 1;
+        a = n2 / d.den;
+        b = n3 / d.den;
+    }
+    qx = a;
+    qy = b;
+    v.x = readlane_r(a, jj);
+    v.y = readlane_r(b, jj);
+}
+
+enum { SOLVE_N, SOLVE_T, SOLVE_LT };
+template <typename R, int MODE, int NR>
+__global__ __launch_bounds__(64)
+void k_gbtrs_reg(int trans, int n, int kl, int ku, int nrhs, const cpx<R> *__restrict__ ab,
+                 int ldab, long long sab, const int *__restrict__ ipiv, long long sipiv,
+                 cpx<R> *__restrict__ b, int ldb, long long sb,
+                 const int *__restrict__ skip, int nsys, const sz::gsys *__restrict__ gs)
+{
+    using T = cpx<R>;
+    constexpr int PF = 8;                    // columns requested ahead
+    extern __shared__ __align__(16) unsigned char smem[];
+    T *xs = reinterpret_cast<T *>(smem);     // n
+    const int sys = blockIdx.x;
+    if (sys >= nsys) return;
+    if (skip && skip[sys] != 0) return;      // singular factor: leave b as is
+    if (gs) {                                // grouped: per-system order, storage
+        const sz::gsys g = gs[sys];
+        n = g.n;
+        ab = reinterpret_cast<const T *>(g.ab);
+        ipiv = reinterpret_cast<const int *>(g.ipiv);
+        b = reinterpret_cast<T *>(g.b);
+    } else {
+        ab += (size_t)sys * (size_t)sab;
+        ipiv += (size_t)sys * (size_t)sipiv;
+        b += (size_t)sys * (size_t)sb;
+    }
+    const int lane = threadIdx.x, kv = kl + ku;
+    const bool cj = trans == 2;
+    // xs[i], zero outside 0 .. n-1
+    auto row = [&](int i, R &x, R &y) __attribute__((always_inline)) {
+        const bool ok = i >= 0 && i < n;
+        const R *v = reinterpret_cast<const R *>(xs + (ok ? i : 0));
+        x = ok ? v[0] : R(0);
+        y = ok ? v[1] : R(0);
+    };
+    // column j, or the nearest there is (its diagonal is loaded and unused)
+    auto col = [&](int j) __attribute__((always_inline)) {
+        return ab + (size_t)max(0, min(j, n - 1)) * ldab;
+    };
+    auto at = [&](const T *c, int i) __attribute__((always_inline)) {
+        return sz::gload(reinterpret_cast<const T *>(reinterpret_cast<const char *>(c) +
+                                                     (unsigned)i * (unsigned)sizeof(T)));
+    };
+    for (int s = 0; s < nrhs; ++s) {
+        T *bs = b + (size_t)s * ldb;
+        for (int i = lane; i < n; i += 64) xs[i] = sz::gload(bs + i);
+        LDS_BARRIER();
+        if constexpr (MODE == SOLVE_N) {
+            // ---- L y = P b
+            if (kl > 0) {
+                R x, y, nx, ny, fx = R(0), fy = R(0), qx[PF], qy[PF];
+                row(lane, x, y);
+                row(64 + lane, nx, ny);
+                // the interchange of step i (LAPACK's last row has none)
+                auto pivot = [&](int i) __attribute__((always_inline)) {
+                    const int c = min(i, n - 1), p = ipiv[c] - 1;
+                    return p < c || p >= n || c == n - 1 ? c : p;
+                };
+                int pv = pivot(lane);
+                // L(j + d, j), d = distance of this lane's row (0: none)
+                auto fetch = [&](int j, R &vx, R &vy) __attribute__((always_inline)) {
+                    const int d = (lane - j) & 63;
+                    const T v = at(col(j), kv + (d <= min(kl, n - 1 - j) ? d : 0));
+                    vx = v.x;
+                    vy = v.y;
+                };
+                unroll<PF>([&](auto u_) __attribute__((always_inline)) {
+                    fetch(decltype(u_)::value, qx[decltype(u_)::value], qy[decltype(u_)::value]);
+                });
+                for (int j0 = 0; j0 < n; j0 += 64) {
+                    for (int jj0 = 0; jj0 < 64 && j0 + jj0 < n; jj0 += PF) {
+                        unroll<PF>([&](auto u_) __attribute__((always_inline)) {
+                            constexpr int u = decltype(u_)::value;
+                            const int jj = jj0 + u, j = j0 + jj;
+                            const int pl = __builtin_amdgcn_readlane(pv, jj) & 63;
+                            const R ax = readlane_r(x, pl), ay = readlane_r(y, pl);
+                            // row p takes row j's value
+                            const R jx = readlane_r(x, jj), jy = readlane_r(y, jj);
+                            x = writelane_r(x, jx, pl);
+                            y = writelane_r(y, jy, pl);
+                            const int d = (lane - jj) & 63;
+                            const bool in = d >= 1 && d <= min(kl, n - 1 - j);
+                            const T v = sz::cfnms(T{x, y}, T{qx[u], qy[u]}, T{ax, ay});
+                            x = sel(in, v.x, x);
+                            y = sel(in, v.y, y);
+                            fx = writelane_r(fx, ax, jj);
+                            fy = writelane_r(fy, ay, jj);
+                            x = sel(d == 0, nx, x);
+                            y = sel(d == 0, ny, y);
+                            __builtin_amdgcn_sched_barrier(0);
+                            fetch(j + PF, qx[u], qy[u]);
+                        });
+                    }
+                    if (j0 + lane < n) xs[j0 + lane] = T{fx, fy};
+                    row(j0 + 128 + lane, nx, ny);
+                    pv = pivot(j0 + 64 + lane);
+                }
+                LDS_BARRIER();
+            }
+            // ---- U x = y, descending; jt: the first column of a block of 64
+            {
+                R x[NR], y[NR], nx, ny, fx = R(0), fy = R(0), qx[PF][NR], qy[PF][NR];
+                const int jl = (n - 1) & 63;
+                const int back = (jl - lane) & 63;     // this lane: row jt - back
+                unroll<NR>([&](auto m_) __attribute__((always_inline)) {
+                    row(n - 1 - back - 64 * decltype(m_)::value, x[decltype(m_)::value],
+                        y[decltype(m_)::value]);
+                });
+                row(n - 1 - back - 64 * NR, nx, ny);
+                // U(j - t, j), t = distance of this lane's rows (t = 0: diagonal)
+                auto fetch = [&](int j, R (&vx)[NR], R (&vy)[NR]) __attribute__((always_inline)) {
+                    const int t0 = (j - lane) & 63;
+                    const T *cp = col(j);
+                    unroll<NR>([&](auto m_) __attribute__((always_inline)) {
+                        constexpr int m = decltype(m_)::value;
+                        const int t = t0 + 64 * m;
+                        const T v = at(cp, kv - (t <= min(kv, j) ? t : 0));
+                        vx[m] = v.x;
+                        vy[m] = v.y;
+                    });
+                };
+                unroll<PF>([&](auto u_) __attribute__((always_inline)) {
+                    fetch(n - 1 - decltype(u_)::value, qx[decltype(u_)::value],
+                          qy[decltype(u_)::value]);
+                });
+                for (int jt = n - 1; jt >= 0; jt -= 64) {
+                    const int dc = max(jt - back, 0);
+                    const T z = sz::gload(ab + (size_t)dc * ldab + kv);
+                    const smith<R> dg = smith_of(z.x, z.y);
+                    for (int k0 = 0; k0 < 64 && k0 <= jt; k0 += PF) {
+                        unroll<PF>([&](auto u_) __attribute__((always_inline)) {
+                            constexpr int u = decltype(u_)::value;
+                            const int j = jt - k0 - u, jj = j & 63;
+                            R wx, wy;
+                            T v;
+                            bool nz;
+                            smith_div(dg, jj, x[0], y[0], wx, wy, v, nz);
+                            const int t0 = (jj - lane) & 63, tl = nz ? min(kv, j) : 0;
+                            unroll<NR>([&](auto m_) __attribute__((always_inline)) {
+                                constexpr int m = decltype(m_)::value;
+                                const int t = t0 + 64 * m;
+                                const T w = sz::cfnms(T{x[m], y[m]}, T{qx[u][m], qy[u][m]}, v);
+                                const bool in = t >= 1 && t <= tl;
+                                x[m] = sel(in, w.x, x[m]);
+                                y[m] = sel(in, w.y, y[m]);
+                            });
+                            const bool done = t0 == 0;   // (0 is left as it is)
+                            fx = sel(done, nz ? wx : x[0], fx);
+                            fy = sel(done, nz ? wy : y[0], fy);
+                            unroll<NR>([&](auto m_) __attribute__((always_inline)) {
+                                constexpr int m = decltype(m_)::value;
+                                R ox = nx, oy = ny;
+                                if constexpr (m + 1 < NR) {
+                                    ox = x[m + 1];
+                                    oy = y[m + 1];
+                                }
+                                x[m] = sel(done, ox, x[m]);
+                                y[m] = sel(done, oy, y[m]);
+                            });
+                            __builtin_amdgcn_sched_barrier(0);
+                            fetch(j - PF, qx[u], qy[u]);
+                        });
+                    }
+                    if (jt - back >= 0) xs[jt - back] = T{fx, fy};
+                    row(jt - 64 - back - 64 * NR, nx, ny);
+                }
+            }
+            LDS_BARRIER();
+        }
+        if constexpr (MODE == SOLVE_T) {
+            // ---- U^T y = b, ascending, four rows a block
+            constexpr int NB = 4, RB = NR == 1 ? 4 : 2;      // RB blocks ahead
+            R x[NR], y[NR], nx, ny, fx = R(0), fy = R(0);
+            R ex[RB][NB][NR], ey[RB][NB][NR];
+            const long long last = (long long)n * ldab - 1;
+            unroll<NR>([&](auto m_) __attribute__((always_inline)) {
+                row(lane + 64 * decltype(m_)::value, x[decltype(m_)::value],
+                    y[decltype(m_)::value]);
+            });
+            row(lane + 64 * NR, nx, ny);
+            // U(jb .. jb+3, c) of this lane's columns c = jb + d + 64 m
+            auto fetch = [&](int jb, R (&vx)[NB][NR], R (&vy)[NB][NR]) __attribute__((always_inline)) {
+                const int d = (lane - jb) & 63;
+                unroll<NR>([&](auto m_) __attribute__((always_inline)) {
+                    constexpr int m = decltype(m_)::value;
+                    const int c = jb + d + 64 * m;
+                    const long long at = (long long)c * ldab + kv - d - 64 * m;
+                    const bool ok = c < n && kv >= d + 64 * m - (NB - 1);
+                    unroll<NB>([&](auto i_) __attribute__((always_inline)) {
+                        constexpr int i = decltype(i_)::value;
+                        const long long k = ok ? at + i : 0;
+                        const T v = sz::gload(ab + (k < 0 ? 0 : k > last ? last : k));
+                        vx[i][m] = v.x;
+                        vy[i][m] = v.y;
+                    });
+                });
+            };
+            unroll<RB>([&](auto h_) __attribute__((always_inline)) {
+                constexpr int h = decltype(h_)::value;
+                fetch(NB * h, ex[h], ey[h]);
+            });
+            for (int j0 = 0; j0 < n; j0 += 64) {
+                const int dc = min(j0 + lane, n - 1);
+                const T z = sz::gload(ab + (size_t)dc * ldab + kv);
+                const smith<R> dg = smith_of(z.x, cj ? -z.y : z.y);
+                for (int jj0 = 0; jj0 < 64 && j0 + jj0 < n; jj0 += RB * NB) {
+                    unroll<RB>([&](auto h_) __attribute__((always_inline)) {
+                        constexpr int h = decltype(h_)::value;
+                        const int jb = j0 + jj0 + NB * h;
+                        const int d = (lane - jb) & 63;
+                        unroll<NB>([&](auto u_) __attribute__((always_inline)) {
+                            constexpr int u = decltype(u_)::value;
+                            const int jj = (jb + u) & 63;
+                            R wx, wy;
+                            T v;
+                            bool nz;
+                            smith_div(dg, jj, x[0], y[0], wx, wy, v, nz);
+                            fx = sel(d == u, wx, fx);
+                            fy = sel(d == u, wy, fy);
+                            unroll<NR>([&](auto m_) __attribute__((always_inline)) {
+                                constexpr int m = decltype(m_)::value;
+                                const int t = d + 64 * m - u;
+                                const T w = sz::cfnms(T{x[m], y[m]},
+                                                      cj_if(T{ex[h][u][m], ey[h][u][m]}, cj),
+                                                      v);
+                                const bool in = t >= 1 && t <= kv;
+                                x[m] = sel(in, w.x, x[m]);
+                                y[m] = sel(in, w.y, y[m]);
+                            });
+                        });
+                        // finished columns' lanes move on by 64
+                        unroll<NR>([&](auto m_) __attribute__((always_inline)) {
+                            constexpr int m = decltype(m_)::value;
+                            R ox = nx, oy = ny;
+                            if constexpr (m + 1 < NR) {
+                                ox = x[m + 1];
+                                oy = y[m + 1];
+                            }
+                            x[m] = sel(d < NB, ox, x[m]);
+                            y[m] = sel(d < NB, oy, y[m]);
+                        });
+                        __builtin_amdgcn_sched_barrier(0);
+                        fetch(jb + RB * NB, ex[h], ey[h]);
+                    });
+                }
+                if (j0 + lane < n) xs[j0 + lane] = T{fx, fy};
+                row(j0 + 64 + 64 * NR + lane, nx, ny);
+            }
+            LDS_BARRIER();
+        }
+        if constexpr (MODE != SOLVE_N) {
+            // ---- L^T x = y and the interchanges, descending.  Lane r holds row
+            // j + 1 + r and forms that row's term of the dot product with
+            // column j's multipliers; the window then moves up by one lane.
+            if (kl > 0 && n > 1) {
+                R x, y, qx[PF], qy[PF];
+                const int back = (n - 2 - lane) & 63;
+                const bool odd = (lane & 1) != 0;
+                row(n - 1 + lane, x, y);
+                // the interchange of step i as the window's lane, -1 for none
+                auto pivot = [&](int i) __attribute__((always_inline)) {
+                    const int c = max(i, 0), p = ipiv[c] - 1;
+                    return p <= c || p >= n || i < 0 ? -1 : p - c - 1;
+                };
+                int pv = pivot(n - 2 - back), npv = pivot(n - 2 - 64 - back);
+                auto fetch = [&](int j, R &vx, R &vy) __attribute__((always_inline)) {
+                    const T v = at(col(j), kv + (lane < min(kl, n - 1 - j) ? 1 + lane : 0));
+                    vx = v.x;
+                    vy = v.y;
+                };
+                unroll<PF>([&](auto u_) __attribute__((always_inline)) {
+                    constexpr int u = decltype(u_)::value;
+                    fetch(n - 2 - u, qx[u], qy[u]);
+                });
+                int j = n - 2;
+                for (int jt = n - 2; jt >= 0; jt -= 64) {
+                    for (int k0 = 0; k0 < 64 && k0 <= jt; k0 += PF) {
+                        // the lanes that PF steps move out of the window (kl <= 56:
+                        // no interchange reaches them any more)
+                        const int i = j + 1 + lane;
+                        if (lane >= 64 - PF && i < n) xs[i] = T{x, y};
+                        R ox[PF], oy[PF];
+                        unroll<PF>([&](auto u_) __attribute__((always_inline)) {
+                            constexpr int u = decltype(u_)::value;
+                            const R *v = reinterpret_cast<const R *>(xs + max(j - u, 0));
+                            ox[u] = v[0];
+                            oy[u] = v[1];
+                        });
+                        unroll<PF>([&](auto u_) __attribute__((always_inline)) {
+                            constexpr int u = decltype(u_)::value;
+                            const bool in = lane < min(kl, n - 1 - j);
+                            const T m = sz::cfma(T{R(0), R(0)}, cj_if(T{qx[u], qy[u]}, cj),
+                                                 T{x, y});
+                            const R acc = wave_csum01(sel(in, m.x, R(0)), sel(in, m.y, R(0)),
+                                                      odd);
+                            R vx = ox[u] - acc, vy = oy[u] - dpp_r<0x55>(acc);  // lane 0
+                            const int p = __builtin_amdgcn_readlane(pv, j & 63);
+                            if (p >= 0) {
+                                const R px = readlane_r(x, p), py = readlane_r(y, p);
+                                x = writelane_r(x, readlane_r(vx, 0), p);
+                                y = writelane_r(y, readlane_r(vy, 0), p);
+                                vx = px;
+                                vy = py;
+                            }
+                            x = wave_shr(x, vx);
+                            y = wave_shr(y, vy);
+                            __builtin_amdgcn_sched_barrier(0);
+                            fetch(j - PF, qx[u], qy[u]);
+                            --j;
+                        });
+                    }
+                    pv = npv;
+                    npv = pivot(jt - 128 - back);
+                }
+                LDS_BARRIER();
+                const int i = j + 1 + lane;
+                if (i >= 0 && i < n) xs[i] = T{x, y};
+            }
+            LDS_BARRIER();
+        }
+        for (int i = lane; i < n; i += 64) sz::gstore(bs + i, xs[i]);
+        LDS_BARRIER();
+    }
+}
 
 // ------------------------------------------------------------ t16 solve
 // A^T x = b (A^H x = b) from the factors, sixteen lanes per system and four
@@ -982,17 +1493,6 @@ __device__ __forceinline__ void fnms_row4(R &ax0, R &ay0, R &ax1, R &ay1, R &ax2
 }
 #undef PN_FOUR
 #undef PN_LINE
-
-template <int... I, typename F>
-__device__ __forceinline__ void unroll_impl(F &&f, std::integer_sequence<int, I...>)
-{
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int K, typename F>
-__device__ __forceinline__ void unroll(F &&f)
-{
-    unroll_impl(f, std::make_integer_sequence<int, K>{});
-}
 
 // One element per lane from p (64 lanes) straight to LDS at dst, without
 // passing through registers: complex doubles as they are, complex floats as
@@ -1805,11 +2305,42 @@ bool launch_gbtrs_t16(int tc, int n, int kl, int ku, const void *ab, int ldab,
     }
 }
 
+// The register solve where the band fits its lanes, else false (k_gbtrs takes
+// any band its staging holds; it is the slower at every band both take, see
+// k_gbtrs_reg).  nmax: the longest right hand side (its LDS).
+template <typename R>
+bool launch_gbtrs_reg(int tc, int n, int kl, int ku, int nrhs, const void *ab, int ldab,
+                      long long sab, const int *ipiv, long long sipiv, void *b, int ldb,
+                      long long sb, const int *skip, int nsys, int nmax,
+                      const sz::gsys *gs, hipStream_t stream, bool lt_only = false)
+{
+    const int kv = kl + ku;
+    // the transposed ones keep finished rows to the end of a block of four (U^T)
+    // and of eight (L^T)
+    if (tc == 0 ? kl > 63 || kv > 127 : kl > 56 || kv > 124) return false;
+    const size_t lds = (size_t)nmax * sizeof(cpx<R>);
+#define SZ_REG(MODE_, NR_)                                                        \
+    hipLaunchKernelGGL((k_gbtrs_reg<R, MODE_, NR_>), dim3(nsys), dim3(64), lds, stream, tc, \
+                       n, kl, ku, nrhs, reinterpret_cast<const cpx<R> *>(ab), ldab, sab, \
+                       ipiv, sipiv, reinterpret_cast<cpx<R> *>(b), ldb, sb, skip, nsys, gs)
+    if (lt_only) {
+        SZ_REG(SOLVE_LT, 1);
+    } else if (tc == 0) {
+        if (kv <= 63) SZ_REG(SOLVE_N, 1);
+        else SZ_REG(SOLVE_N, 2);
+    } else {
+        if (kv <= 60) SZ_REG(SOLVE_T, 1);
+        else SZ_REG(SOLVE_T, 2);
+    }
+#undef SZ_REG
+    return true;
+}
+
 template <typename R>
 int launch_gbtrs(char trans, int n, int kl, int ku, int nrhs, const void *ab,
                  int ldab, long long sab, const int *ipiv, long long sipiv,
                  void *b, int ldb, long long sb, const int *skip, int nsys,
-                 hipStream_t stream, int skip_ut = 0)
+                 hipStream_t stream, bool lt_only = false)
 {
     const int tc = trans_code(trans);
     if (tc < 0) return -1;
@@ -1831,25 +2362,24 @@ int launch_gbtrs(char trans, int n, int kl, int ku, int nrhs, const void *ab,
                                      + 64 * sizeof(int)
                                : (size_t)n * sizeof(cpx<R>);
     if (lds > LDS_MAX) return SZ_ERR_LDS;
-    if (nrhs == 1 && !skip_ut &&
+    if (nrhs == 1 && !lt_only &&
         launch_gbtrs_t16<R>(tc, n, kl, ku, ab, ldab, sab, ipiv, sipiv, b, sb, skip,
                             nsys, n, nullptr, stream))
         return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
+    if (launch_gbtrs_reg<R>(tc, n, kl, ku, nrhs, ab, ldab, sab, ipiv, sipiv, b, ldb, sb,
+                            skip, nsys, n, nullptr, stream, lt_only))
+        return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
+    if (lt_only) return SZ_ERR_LDS;          // only after a fused factorization
     if (tc == 0)
         hipLaunchKernelGGL((k_gbtrs<R, false>), dim3(nsys), dim3(TRS_NT), lds, stream, tc, n,
                        kl, ku, nrhs, reinterpret_cast<const cpx<R> *>(ab), ldab,
                        sab, ipiv, sipiv, reinterpret_cast<cpx<R> *>(b), ldb, sb,
-                       skip, nsys, skip_ut);
-    else if (skip_ut)
-        hipLaunchKernelGGL((k_gbtrs<R, true, true>), dim3(nsys), dim3(TRS_NT), lds, stream, tc, n,
-                       kl, ku, nrhs, reinterpret_cast<const cpx<R> *>(ab), ldab,
-                       sab, ipiv, sipiv, reinterpret_cast<cpx<R> *>(b), ldb, sb,
-                       skip, nsys, skip_ut);
+                       skip, nsys);
     else
         hipLaunchKernelGGL((k_gbtrs<R, true>), dim3(nsys), dim3(TRS_NT), lds, stream, tc, n,
                        kl, ku, nrhs, reinterpret_cast<const cpx<R> *>(ab), ldab,
                        sab, ipiv, sipiv, reinterpret_cast<cpx<R> *>(b), ldb, sb,
-                       skip, nsys, skip_ut);
+                       skip, nsys);
     return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
 }
 
@@ -1932,10 +2462,13 @@ int launch_gbtrs_grouped(char trans, int kl, int ku, const void *ab, int ldab,
     if (launch_gbtrs_t16<R>(tc, 0, kl, ku, ab, ldab, 0LL, ipiv, 0LL, b, 0LL, skip, nsys,
                             nmax, gs, stream))
         return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
+    if (launch_gbtrs_reg<R>(tc, 0, kl, ku, 1, ab, ldab, 0LL, ipiv, 0LL, b, nmax, 0LL, skip,
+                            nsys, nmax, gs, stream))
+        return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
     hipLaunchKernelGGL((k_gbtrs<R, true>), dim3(nsys), dim3(TRS_NT), lds, stream, tc,
                        nmax, kl, ku, 1, reinterpret_cast<const cpx<R> *>(ab), ldab,
                        0LL, ipiv, 0LL, reinterpret_cast<cpx<R> *>(b), nmax, 0LL, skip,
-                       nsys, 0, gs);
+                       nsys, gs);
     return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
 }
 
@@ -2048,7 +2581,7 @@ int sz_internal_zgbtrs_lt(int n, int kl, int ku, const void *ab, int ldab,
 {
     return launch_gbtrs<double>('T', n, kl, ku, 1, ab, ldab, strideab, ipiv,
                                 strideipiv, b, n, strideb, skip, nbatch,
-                                (hipStream_t)stream, 1);
+                                (hipStream_t)stream, true);
 }
 
 int sz_internal_gbtrf_masked(int single, int n, int kl, int ku, void *ab,
