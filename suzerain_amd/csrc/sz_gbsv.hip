@@ -609,7 +609,7 @@ void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
 // systems by issue of the SIMD; the factors' bytes take a third of the time.
 // Measured, against x in LDS with a barrier a step: N of 576 systems n = 480,
 // kl = ku = 34: 459 -> 294 us (455 MB); T of 600 systems n = 301, kl 17, ku 11,
-// two right hand sides: 615 -> 253 us; L^T of 1520 systems n = 480, kl = 34:
+// two right hand sides: 615 -> 253 us; L^T of 4560 systems n = 480, kl = 34:
 // 483 -> 334 us; N in float, 300 systems n = 200, kl = ku = 24: 37 -> 19 us.
 template <typename R>
 __device__ __forceinline__ R sel(bool c, R a, R b) { return c ? a : b; }

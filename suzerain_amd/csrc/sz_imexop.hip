@@ -27,6 +27,8 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -178,6 +180,45 @@ void build_table(const double *sc, table &tab)
     tab.ngroups = ng;
 }
 
+// The table's structure, which no scenario changes: with it as constants the
+// apply kernels unroll every block, group and term.  shape_ok() holds a built
+// table against it.
+constexpr int NTERM = 96, NGROUP = 50;
+constexpr int BG0[25] = {0, 3, 6, 9, 12, 16, 17, 20, 22, 23, 26, 27, 29, 32, 34,
+                         37, 38, 39, 41, 44, 47, 47, 48, 49, 50};
+constexpr int BNG[25] = {3, 3, 3, 3, 4, 1, 3, 2, 1, 3, 1, 2, 3, 2, 3,
+                         1, 1, 2, 3, 3, 0, 1, 1, 1, 0};
+constexpr int GOP[NGROUP] = {0, 1, 2, 0, 1, 2, 0, 1, 2, 0, 1, 2, 0, 0, 1, 2, 0,
+                             0, 1, 2, 0, 1, 0, 0, 1, 2, 1, 0, 1, 0, 1, 2, 0, 1,
+                             0, 1, 2, 0, 0, 0, 1, 0, 1, 2, 0, 1, 2, 0, 1, 0};
+constexpr int GT0[NGROUP] = {0, 3, 4, 5, 8, 9, 10, 11, 14, 15, 18, 19, 20, 24, 27,
+                             30, 33, 34, 37, 38, 39, 40, 42, 45, 50, 52, 53, 54, 55,
+                             57, 60, 61, 62, 63, 65, 68, 72, 73, 74, 77, 78, 80, 83,
+                             84, 85, 90, 92, 93, 94, 95};
+constexpr int GNT[NGROUP] = {3, 1, 1, 3, 1, 1, 1, 3, 1, 3, 1, 1, 4, 3, 3, 3, 1,
+                             3, 1, 1, 1, 2, 3, 5, 2, 1, 1, 1, 2, 3, 1, 1, 1, 2,
+                             3, 4, 1, 1, 3, 1, 2, 3, 1, 1, 5, 2, 1, 1, 1, 1};
+constexpr int TREF[NTERM] = {
+    ux, uz, nu, uy, nu, nuux, nuuz, e_divm, nuuy, nuux, nuuy, nuux, nuuz, e_divm,
+    nuuy, nuux, nuuz, e_divm, nuuy, nuuz, nuu2, nuuxux, nuuxuz, nuuzuz, ex_gradrho,
+    ez_gradrho, e_deltarho, nuuxuy, nuuyuz, ey_gradrho, nuu2, nuuyuy, e_deltarho,
+    ONE, ux, uz, nu, uy, nu, uy, ux, nu, ux, uz, nu, u2, uxux, uxuz, nuux, nuuz,
+    uxuy, nuuy, nuux, ONE, uy, ux, nu, ux, uz, nu, uy, nu, uy, uz, nu, uxuy, uyuz,
+    nuuy, u2, uyuy, nuux, nuuz, nuuy, ONE, ux, uz, nu, uy, uz, nu, ux, uz, nu, uy,
+    nu, u2, uxuz, uzuz, nuuz, nuux, uyuz, nuuy, nuuz, ONE, ONE, ONE};
+
+template <int N, size_t M>
+bool same(const int (&a)[M], const int (&b)[N])
+{
+    return std::equal(b, b + N, a);
+}
+bool shape_ok(const table &t)
+{
+    return t.nterms == NTERM && t.ngroups == NGROUP && same(t.bg0, BG0) &&
+           same(t.bng, BNG) && same(t.gop, GOP) && same(t.gt0, GT0) &&
+           same(t.gnt, GNT) && same(t.tref, TREF);
+}
+
 __device__ inline zd kappa(const double *k, double km, double kn)
 {
     const double km2 = km * km, kn2 = kn * kn, kmkn = km * kn;
@@ -226,30 +267,9 @@ __device__ inline zd weight_staged(const int *gt0, const int *gnt, const int *tr
     return zd{wx, wy};
 }
 
-// weight_staged with the reference values staged in LDS, refl[q * n + r] =
-// ref_q[r]: the same arithmetic without a global gather per term.
-__device__ inline zd weight_lds(const int *gt0, const int *gnt, const int *tref,
-                                const double *refl, int n, const zd *alpha, int g,
-                                int r)
-{
-    const int t0 = gt0[g], nt = gnt[g];
-    double wx = 0, wy = 0;
-    for (int q = 0; q < nt; ++q) {
-        const int t = t0 + q, rt = tref[t];
-        const double v = rt == ONE ? 1.0 : refl[rt * n + r];
-        if (q == 0) {
-            wx = alpha[t].x * v;
-            wy = alpha[t].y * v;
-        } else {
-            wx = fma(alpha[t].x, v, wx);
-            wy = fma(alpha[t].y, v, wy);
-        }
-    }
-    return zd{wx, wy};
-}
-
 struct bops {
     const double *dt;     // derivative d's transposed band at dt + d * dstride
+    const double *dc;     // its rows' element t (from 0) for every row: dc[(3 t + d) n + r]
     long long dstride;
     int n, ld, max_kl, max_ku;
     int kl[3], ku[3];
@@ -260,44 +280,157 @@ struct wallbc {
     double fac[2][4];     // E_factor, u, v, w per wall
 };
 
-// refl[q * n + y] = ref_q[y] for every point y (0 for an absent profile),
-// from the profile columns rp/rld already staged in LDS; the block's
-// threads share the 26n loads (a few each).
-template <int NTH>
-__device__ __forceinline__ void stage_refs(const double *const *rp, const int *rld,
-                                           int n, double *refl)
+template <int... I, typename F>
+__device__ __forceinline__ void each_impl(F &f, std::integer_sequence<int, I...>)
 {
-    for (int e = threadIdx.x; e < NREF * n; e += NTH) {
-        const int q = e / n, y = e - q * n;
-        const double *p = rp[q];
-        refl[e] = p ? *sz::gmem(p + (long long)y * rld[q]) : 0.0;
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void each(F &&f)
+{
+    each_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// refl[q * n + y] = ref_q[y] for every point y (0 for an absent profile); the
+// block's threads share the 26n loads (a few each).  Nothing may read refl or
+// srp before the caller's next barrier.
+template <int NTH>
+__device__ __forceinline__ void stage_refs(const refs &rf, int n, const double **srp,
+                                           int *srld, double *refl)
+{
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int q = 0; q < NREF; ++q) {        // static indices: no private copy
+            srp[q] = rf.p[q];
+            srld[q] = rf.ld[q];
+        }
+    }
+    __syncthreads();
+    constexpr int U = 8;                        // loads in flight a thread
+    for (int e0 = threadIdx.x; e0 < NREF * n; e0 += U * NTH) {
+        double v[U];
+        each<U>([&](auto u_) __attribute__((always_inline)) {
+            constexpr int u = decltype(u_)::value;
+            const int e = min(e0 + u * NTH, NREF * n - 1), q = e / n, y = e - q * n;
+            const double *p = srp[q];
+            v[u] = p ? *sz::gmem(p + (long long)y * srld[q]) : 0.0;
+        });
+        each<U>([&](auto u_) __attribute__((always_inline)) {
+            constexpr int u = decltype(u_)::value;
+            if (e0 + u * NTH < NREF * n) refl[e0 + u * NTH] = v[u];
+        });
     }
 }
 
-// The band products of operator op at wall-normal point r for all five
-// fields: Dx[(op * 5 + f) * n + r] = sum over the band columns c (ascending,
-// a fused multiply-add per term from zero) of D_T(r, c) x_f[c], x_f at
-// xs + f n.  Each coefficient is loaded once for the five fields.
-__device__ __forceinline__ void band_products5(const bops &w, int op, int r,
-                                               const zd *xs, zd *Dx)
+// Row r of (M + phi L) x for one system by one thread: emit(i, L part, M x_i)
+// for the five equations.  xs holds the system's five fields, max_ku zeros
+// before and max_kl after each (a band sticking out of the matrix multiplies
+// them: no bound to test), al its NTERM weights phi kappa_t, refl the reference
+// profiles, all in LDS.  Not ALL: only the fields and equations in mask.
+// The block, group and term loops unroll on the constant structure: a weight
+// costs one broadcast read of LDS and two multiply-adds, a profile value is read
+// once for the row, and no index passes through memory.  Each x value is read
+// once for the three operators; their coefficients are contiguous over the rows
+// (a row's own run, strided over the lanes, touches a cache line a lane).
+template <bool ALL, typename F>
+__device__ __forceinline__ void op_rows(const bops &w, int r, const zd *xs, const zd *al,
+                                        const double *refl, unsigned mask, F &&emit)
 {
-    const int n = w.n;
-    const double *row = w.dt + op * w.dstride + (long long)r * w.ld + w.max_ku - r;
-    double tx[5], ty[5];
-#pragma unroll
-    for (int f = 0; f < 5; ++f) tx[f] = ty[f] = 0;
-    const int c1 = min(n - 1, r + w.kl[op]);
-    for (int c = max(0, r - w.ku[op]); c <= c1; ++c) {
-        const double a = *sz::gmem(row + c);
-#pragma unroll
-        for (int f = 0; f < 5; ++f) {
-            const zd xv = xs[f * n + c];
-            tx[f] = fma(a, xv.x, tx[f]);
-            ty[f] = fma(a, xv.y, ty[f]);
+    const int n = w.n, hi = w.max_kl, fs = n + w.max_kl + w.max_ku;
+    double dx[15], dy[15];                          // operator op, field f: 5 op + f
+    each<15>([&](auto k_) __attribute__((always_inline)) {
+        dx[decltype(k_)::value] = dy[decltype(k_)::value] = 0;
+    });
+    auto fetch = [&](int t, double (&a)[3]) __attribute__((always_inline)) {
+        const double *p = w.dc + (long long)(min(t, hi) + w.max_ku) * 3 * n;
+        each<3>([&](auto o_) __attribute__((always_inline)) {
+            constexpr int op = decltype(o_)::value;
+            a[op] = sz::gmem(p + op * n)[(unsigned)r];
+        });
+    };
+    auto products = [&](auto full) __attribute__((always_inline)) {
+        double a[3];
+        fetch(-w.max_ku, a);
+#pragma unroll 2
+        for (int t = -w.max_ku; t <= hi; ++t) {
+            double next[3], vx[5], vy[5];
+            fetch(t + 1, next);
+            each<5>([&](auto f_) __attribute__((always_inline)) {
+                constexpr int f = decltype(f_)::value;
+                const double *v = reinterpret_cast<const double *>(xs + f * fs + r + t);
+                vx[f] = v[0];
+                vy[f] = v[1];
+            });
+            each<3>([&](auto o_) __attribute__((always_inline)) {
+                constexpr int op = decltype(o_)::value;
+                if (decltype(full)::value || (t >= -w.ku[op] && t <= w.kl[op]))
+                    each<5>([&](auto f_) __attribute__((always_inline)) {
+                        constexpr int f = decltype(f_)::value, k = 5 * op + f;
+                        dx[k] = fma(a[op], vx[f], dx[k]);
+                        dy[k] = fma(a[op], vy[f], dy[k]);
+                    });
+            });
+            each<3>([&](auto o_) __attribute__((always_inline)) {
+                a[decltype(o_)::value] = next[decltype(o_)::value];
+            });
         }
-    }
-#pragma unroll
-    for (int f = 0; f < 5; ++f) Dx[(op * 5 + f) * n + r] = zd{tx[f], ty[f]};
+    };
+    bool full = true;
+    each<3>([&](auto o_) __attribute__((always_inline)) {
+        constexpr int op = decltype(o_)::value;
+        full = full && w.ku[op] == w.max_ku && w.kl[op] == w.max_kl;
+    });
+    if (full) products(std::true_type{});
+    else products(std::false_type{});
+    each<5>([&](auto i_) __attribute__((always_inline)) {
+        constexpr int i = decltype(i_)::value;
+        if (!ALL && !(mask >> i & 1)) return;
+        // the profiles are read again for every equation: kept, with the
+        // products, they would not fit the registers
+        int rr = r;
+        asm volatile("" : "+v"(rr));
+        zd acc{0, 0};
+        each<5>([&](auto j_) __attribute__((always_inline)) {
+            constexpr int j = decltype(j_)::value, blk = 5 * i + j;
+            if (!ALL && !(mask >> j & 1)) return;
+            each<BNG[blk]>([&](auto g_) __attribute__((always_inline)) {
+                constexpr int g = BG0[blk] + decltype(g_)::value, k = 5 * GOP[g] + j;
+                double wx = 0, wy = 0;
+                each<GNT[g]>([&](auto t_) __attribute__((always_inline)) {
+                    constexpr int t = GT0[g] + decltype(t_)::value, q = TREF[t];
+                    double v = 1.0;
+                    if constexpr (q >= 0) v = refl[q * n + rr];
+                    const double *av = reinterpret_cast<const double *>(al + t);
+                    if constexpr (decltype(t_)::value == 0) {
+                        wx = av[0] * v;
+                        wy = av[1] * v;
+                    } else {
+                        wx = fma(av[0], v, wx);
+                        wy = fma(av[1], v, wy);
+                    }
+                });
+                acc = sz::cfma(acc, zd{wx, wy}, zd{dx[k], dy[k]});
+            });
+            // (orders the blocks: all their loads first would not fit)
+            asm volatile("" : "+v"(acc.x), "+v"(acc.y) :: "memory");
+        });
+        emit(i_, acc, zd{dx[i], dy[i]});
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+
+// LDS of an apply block: the profiles, then per system its term weights and
+// five fields.
+__host__ __device__ constexpr size_t ap_refs(int n) { return sizeof(double) * NREF * (size_t)n; }
+__host__ __device__ constexpr size_t ap_slot(int n, int pad)    // pad: max_kl + max_ku
+{
+    return sizeof(zd) * (NTERM + 5 * (size_t)(n + pad));
+}
+// the zeros around field f, a few by each of the system's n threads
+__device__ __forceinline__ void ap_margins(const bops &w, int r, zd *xf)
+{
+    for (int e = r; e < w.max_ku; e += w.n) xf[-1 - e] = zd{0, 0};
+    for (int e = r; e < w.max_kl; e += w.n) xf[w.n + e] = zd{0, 0};
 }
 
 constexpr int PK_NT = 256;
@@ -582,288 +715,261 @@ void k_imexop_pack_listed(const gmember *__restrict__ mem, int nm,
     }
 }
 
-// the x, D x buffers take most of a CU's LDS (one workgroup per CU), so the
-// workgroup is large enough to hide the latency of its own loads
-constexpr int AC_NT = 1024;
-// LDS of the reference profiles staged at every point (order n), which the
-// accumulate and apply kernels use when they have room for it (the sweep
-// keeps the gather: the extra LDS would cost it a resident workgroup).
-#define REFL_BYTES(n) (sizeof(double) * NREF * (size_t)(n))
+// Threads of an apply block: a thread takes one wall-normal row of one of the
+// block's systems.  Two blocks of AP_NT stay on a CU where their LDS fits, so
+// one loads while the other computes; else one of AP_NT1 (see apply_blocks).
+// Bound by latency at three waves a SIMD (the 1,150 instructions of a row are
+// a third of the time, the bytes a third to a half).  Measured, against one
+// system a block of 1,024 threads with weights formed from tables in LDS: 4,560
+// systems n = 96 130 -> 77 us (0.36 GB), 18,336 systems n = 192 1080 -> 485 us
+// and their refinement sweep 840 -> 406 us; of which 840 -> 490 by the constant
+// structure, the rest by y and b requested before the products.
+constexpr int AP_NT = 384, AP_NT1 = 768;
+#define AP_BOUNDS(NT_) __launch_bounds__(NT_) __attribute__((amdgpu_waves_per_eu(3, 3)))
 
-// y_i <- (M + phi L) x + beta y_i for the systems s = blockIdx.x,
-// blockIdx.x + gridDim.x, ... < nsys (those with skip[s] != 0 left alone).
+struct fields {
+    const zd *in[5];
+    zd *out[5];
+};
+
+// y_i <- (M + phi L) x + beta y_i for the systems s < nsys (those with
+// skip[s] != 0 left alone), slots at a time, blocks striding over them.
 // Field f of system s starts at in_f + inoff(s) (complex elements, stride 1
-// in y; a null in_f is an absent field).  A block stages the operator's
-// term tables (and, STAGED, the reference profiles at every point) once and
-// keeps them for all of its systems; per system it computes the term
-// weights of its wavenumbers, the 15 band products D x and the outputs.
-template <bool STAGED>
-__global__ __launch_bounds__(AC_NT) __attribute__((amdgpu_waves_per_eu(8)))
+// in y); not ALL: absent fields are null.  A block stages the reference
+// profiles once and keeps them for all of its systems.
+template <bool ALL, int NTH>
+__global__ AP_BOUNDS(NTH)
 void k_imexop_accumulate(const table *__restrict__ tab, bops w, refs rf, zd phi,
-                         const double *__restrict__ km,
-                         const double *__restrict__ kn, const zd *in0,
-                         const zd *in1, const zd *in2, const zd *in3,
-                         const zd *in4, const long long *__restrict__ inoff,
-                         long long instride, zd beta, int beta_zero, zd *out0,
-                         zd *out1, zd *out2, zd *out3, zd *out4,
-                         const long long *__restrict__ outoff,
-                         long long outstride, const int *__restrict__ skip,
-                         int nsys)
+                         const double *__restrict__ km, const double *__restrict__ kn,
+                         fields F, const long long *__restrict__ inoff,
+                         long long instride, zd beta, int beta_zero,
+                         const long long *__restrict__ outoff, long long outstride,
+                         const int *__restrict__ skip, int nsys, int slots)
 {
-    extern __shared__ double smem[];
-    const int n = w.n;
-    zd *alpha = reinterpret_cast<zd *>(smem);       // MAXTERMS
-    zd *xs = alpha + MAXTERMS;                      // 5 x n
-    zd *Dx = xs + 5 * n;                            // 3 x 5 x n
-    double *refl = reinterpret_cast<double *>(Dx + 15 * n);   // NREF x n if STAGED
-    __shared__ int sbg0[25], sbng[25], sgop[MAXGROUPS], sgt0[MAXGROUPS], sgnt[MAXGROUPS];
-    __shared__ int stref[MAXTERMS], srld[NREF];
+    extern __shared__ __align__(16) unsigned char apmem[];
     __shared__ const double *srp[NREF];
-    {
-        const int tid = threadIdx.x;
-        for (int t = tid; t < tab->nterms; t += AC_NT) stref[t] = tab->tref[t];
-        for (int g = tid; g < tab->ngroups; g += AC_NT) {
-            sgop[g] = tab->gop[g];
-            sgt0[g] = tab->gt0[g];
-            sgnt[g] = tab->gnt[g];
-        }
-        if (tid < 25) {
-            sbg0[tid] = tab->bg0[tid];
-            sbng[tid] = tab->bng[tid];
-        }
-        if (tid == 0) {
-#pragma unroll
-            for (int q = 0; q < NREF; ++q) {    // static indices: no private copy
-                srp[q] = rf.p[q];
-                srld[q] = rf.ld[q];
-            }
-        }
-    }
-    __syncthreads();
-    if constexpr (STAGED) stage_refs<AC_NT>(srp, srld, n, refl);
-    const zd *const inb[5] = {in0, in1, in2, in3, in4};
-    zd *const outb[5] = {out0, out1, out2, out3, out4};
-    for (int s = blockIdx.x; s < nsys; s += gridDim.x) {
-        __syncthreads();        // the previous system's LDS is read out
-        if (skip && skip[s]) continue;           // uniform over the block
+    __shared__ int srld[NREF];
+    const int n = w.n;
+    double *refl = reinterpret_cast<double *>(apmem);            // NREF x n
+    zd *al = reinterpret_cast<zd *>(apmem + (ap_refs(n) + 15) / 16 * 16);
+    const int fs = n + w.max_kl + w.max_ku;
+    zd *xs = al + slots * NTERM + w.max_ku;                     // slots x 5 x fs
+    stage_refs<NTH>(rf, n, srp, srld, refl);
+    unsigned mask = 0;
+    each<5>([&](auto f_) __attribute__((always_inline)) {
+        constexpr int f = decltype(f_)::value;
+        if (ALL || F.in[f]) mask |= 1u << f;
+    });
+    for (int s0 = blockIdx.x * slots; s0 < nsys; s0 += gridDim.x * slots) {
         // the thread index as a value the compiler cannot hold across
-        // systems: what it derives is recomputed per system instead of
-        // occupying registers through the whole loop
+        // systems: what it derives is recomputed instead of occupying
+        // registers through the whole loop
         int tid = threadIdx.x;
         asm volatile("" : "+v"(tid));
-        const long long io = inoff ? inoff[s] : (long long)s * instride;
-        const long long oo = outoff ? outoff[s] : (long long)s * outstride;
-        const double kms = km[s], kns = kn[s];
-        for (int t = tid; t < tab->nterms; t += AC_NT)
-            alpha[t] = sz::cmul(phi, kappa(tab->tk[t], kms, kns));
-        for (int e = tid; e < 5 * n; e += AC_NT) {
-            const int f = e / n, y = e - f * n;
-            xs[e] = inb[f] ? sz::gload(inb[f] + io + y) : zd{0, 0};
+        const int slot = tid / n, r = tid - slot * n, s = s0 + slot;
+        const bool act = slot < slots && s < nsys && !(skip && skip[s]);
+        __syncthreads();        // the previous systems' LDS is read out
+        for (int e = tid; e < slots * NTERM; e += NTH) {
+            const int q = e / NTERM, t = e - q * NTERM, sq = s0 + q;
+            if (sq < nsys) al[e] = sz::cmul(phi, kappa(tab->tk[t], km[sq], kn[sq]));
+        }
+        if (act) {
+            const long long io = inoff ? inoff[s] : (long long)s * instride;
+            each<5>([&](auto f_) __attribute__((always_inline)) {
+                constexpr int f = decltype(f_)::value;
+                zd *xf = xs + (slot * 5 + f) * fs;
+                xf[r] = ALL || F.in[f] ? sz::gload(F.in[f] + io + r) : zd{0, 0};
+                ap_margins(w, r, xf);
+            });
         }
         __syncthreads();
-        for (int e = tid; e < 3 * n; e += AC_NT)
-            band_products5(w, e / n, e % n, xs, Dx);
-        __syncthreads();
-        for (int e = tid; e < 5 * n; e += AC_NT) {
-            const int i = e / n, r = e - i * n;
-            if (!outb[i]) continue;
-            zd acc{0, 0};
-            for (int j = 0; j < 5; ++j) {
-                if (!inb[j]) continue;
-                const int b = i * 5 + j, g0 = sbg0[b], ng = sbng[b];
-                for (int g = g0; g < g0 + ng; ++g) {
-                    const zd W = STAGED ? weight_lds(sgt0, sgnt, stref, refl, n, alpha, g, r)
-                                        : weight_staged(sgt0, sgnt, stref, srp, srld, alpha, g, r);
-                    acc = sz::cfma(acc, W, Dx[(sgop[g] * 5 + j) * n + r]);
+        if (act) {
+            const long long oo = (outoff ? outoff[s] : (long long)s * outstride) + r;
+            double yx[5], yy[5];                    // requested before the products
+            each<5>([&](auto f_) __attribute__((always_inline)) {
+                constexpr int f = decltype(f_)::value;
+                yx[f] = yy[f] = 0;
+                if (!beta_zero && (ALL || F.out[f])) {
+                    const zd v = sz::gload(F.out[f] + oo);
+                    yx[f] = v.x;
+                    yy[f] = v.y;
                 }
-            }
-            zd *yp = outb[i] + oo + r;
-            zd by = beta_zero ? zd{0, 0} : sz::cmul(beta, sz::gload(yp));
-            const zd sm{by.x + acc.x, by.y + acc.y};
-            const zd m = Dx[(M * 5 + i) * n + r];
-            sz::gstore(yp, zd{sm.x + m.x, sm.y + m.y});
+            });
+            op_rows<ALL>(w, r, xs + slot * 5 * fs, al + slot * NTERM, refl, mask,
+                         [&](auto i_, zd acc, zd m) __attribute__((always_inline)) {
+                constexpr int i = decltype(i_)::value;
+                zd *yp = F.out[i] + oo;
+                const zd by = beta_zero ? zd{0, 0} : sz::cmul(beta, zd{yx[i], yy[i]});
+                const zd sm{by.x + acc.x, by.y + acc.y};
+                sz::gstore(yp, zd{sm.x + m.x, sm.y + m.y});
+            });
         }
     }
 }
 
-// Block sum (AC_NT threads, tid = the thread index); every thread gets it.
-__device__ __forceinline__ double block_sum_ac(double v, double *red, int tid)
-{
-    const int lane = tid & 63;
-    for (int off = 32; off >= 1; off >>= 1) v += xor_lane(v, lane, off);
-    const int w = tid >> 6;
-    __syncthreads();
-    if (lane == 0) red[w] = v;
-    __syncthreads();
-    double t = 0;
-    for (int i = 0; i < AC_NT / 64; ++i) t += red[i];
-    return t;
-}
-
-// One refinement sweep of the mixed precision solve for global system s,
-// member-local index ls, by the whole block: x += P^T c (c the float
+// One refinement sweep of the mixed precision solve over the systems
+// a.list[0 .. *a.count) (global indices, any order): x += P^T c (c the float
 // correction in a.PB), r = b - (M + phi L) x with the isothermal wall rows
 // evaluated as the constraints s (x_f - fac x_rho) = 0 whose scalings s the
 // factors hold, ||r||_2 and ||x||_2, the decision of dsgbsvx.def:186-227,
 // and for the systems that continue the next right hand side P r in float.
-// The operator product is the accumulate body's arithmetic, with the
-// member's reference profiles in LDS when PROF (staged when stage is set:
-// the block's previous system belonged to another member), else gathered.
-// Returns the system's new state (the same in every thread).
-template <bool PROF>
-__device__ __forceinline__ int sweep_body(const gmember &M, int ls, int s,
-                                          const sz_prec_sweep &a, int tid, bool stage)
+// Each block takes a contiguous share of the list, as many neighbours of one
+// member at a time as its LDS holds (lds bytes); the profiles are staged when
+// the member changes.  A norm is summed by 16 partial sums a system, an order
+// that depends on n alone.  Continuing systems are collected in LDS and
+// appended to a.next (count *a.ncount, cleared by the caller) with one atomic a
+// block, so that sweeps after convergence cost a handful of blocks.
+template <int NTH>
+__global__ AP_BOUNDS(NTH)
+void k_imexop_sweep_listed(const gmember *__restrict__ mem, int nm, sz_prec_sweep a,
+                           int lds)
 {
-    extern __shared__ double smem[];
-    const table *__restrict__ tab = M.tab;
-    const bops &w = M.w;
-    const refs &rf = M.rf;
-    const int n = w.n, N = 5 * n;
-    zd *alpha = reinterpret_cast<zd *>(smem);       // MAXTERMS
-    zd *xs = alpha + MAXTERMS;                      // 5 x n
-    zd *Dx = xs + 5 * n;                            // 3 x 5 x n
-    zd *rr = Dx + 15 * n;                           // 5 x n
-    double *refl = reinterpret_cast<double *>(rr + 5 * n);   // NREF x n
-    __shared__ int sbg0[25], sbng[25], sgop[MAXGROUPS], sgt0[MAXGROUPS], sgnt[MAXGROUPS];
-    __shared__ int stref[MAXTERMS], srld[NREF];
+    constexpr int NPEND = 256, G = 16, MAXSLOT = 64;
+    extern __shared__ __align__(16) unsigned char apmem[];
     __shared__ const double *srp[NREF];
-    __shared__ double red[AC_NT / 64];
-    const long long o = M.v0 + (long long)ls * N;
-    zd *x = a.X + o;
-    const zd *b = a.B + o;
-    sz::zf *pb = a.PB + o;
-    // read before the barriers: thread 0 rewrites the state at the end
-    sz_psys S = a.S[s];
-    const int apprx = M.apprx[ls];
-    const double kms = M.km[ls], kns = M.kn[ls];
-    for (int t = tid; t < tab->nterms; t += AC_NT) {
-        alpha[t] = sz::cmul(M.phi, kappa(tab->tk[t], kms, kns));
-        stref[t] = tab->tref[t];
-    }
-    for (int g = tid; g < tab->ngroups; g += AC_NT) {
-        sgop[g] = tab->gop[g];
-        sgt0[g] = tab->gt0[g];
-        sgnt[g] = tab->gnt[g];
-    }
-    if (tid < 25) {
-        sbg0[tid] = tab->bg0[tid];
-        sbng[tid] = tab->bng[tid];
-    }
-    if (tid == 0) {
-#pragma unroll
-        for (int q = 0; q < NREF; ++q) {        // static indices: no private copy
-            srp[q] = rf.p[q];
-            srld[q] = rf.ld[q];
-        }
-    }
-    for (int e = tid; e < N; e += AC_NT) {
-        const int f = e / n, y = e - f * n;
-        const sz::zf c = sz::gload(pb + y * 5 + f);   // (P^T c)_e = c_{q^-1(e)}
-        const zd xo = a.first ? zd{0, 0} : sz::gload(x + e);
-        const zd v = zd{xo.x + (double)c.x, xo.y + (double)c.y};
-        xs[e] = v;
-        sz::gstore(x + e, v);
-    }
-    __syncthreads();
-    if (PROF && stage) stage_refs<AC_NT>(srp, srld, n, refl);
-    for (int e = tid; e < 3 * n; e += AC_NT)
-        band_products5(w, e / n, e % n, xs, Dx);
-    __syncthreads();
-    double ss = 0, xx = 0;
-    for (int e = tid; e < N; e += AC_NT) {
-        const int i = e / n, r = e - i * n;
-        const int wall = r == 0 ? 0 : (r == n - 1 ? 1 : -1);
-        zd v;
-        if (i < 4 && wall >= 0 && M.bc.enforce[wall]) {
-            const zd sc = sz::gload(M.bcs + (size_t)ls * 8 + wall * 4 + i);
-            const double fac = M.bc.fac[wall][i];
-            const zd xr = xs[4 * n + r];
-            const zd c = zd{xs[e].x - fac * xr.x, xs[e].y - fac * xr.y};
-            const zd p = sz::cmul(sc, c);
-            v = zd{-p.x, -p.y};
-        } else {
-            zd acc{0, 0};
-            for (int j = 0; j < 5; ++j) {
-                const int bb = i * 5 + j, g0 = sbg0[bb], ng = sbng[bb];
-                for (int g = g0; g < g0 + ng; ++g) {
-                    const zd W = PROF ? weight_lds(sgt0, sgnt, stref, refl, n, alpha, g, r)
-                                      : weight_staged(sgt0, sgnt, stref, srp, srld, alpha, g, r);
-                    acc = sz::cfma(acc, W, Dx[(sgop[g] * 5 + j) * n + r]);
-                }
-            }
-            const zd m = Dx[(0 * 5 + i) * n + r];    // the mass operator M
-            const zd t = zd{acc.x + m.x, acc.y + m.y};
-            const zd be = sz::gload(b + e);
-            v = zd{be.x - t.x, be.y - t.y};
-        }
-        rr[e] = v;
-        ss += v.x * v.x + v.y * v.y;
-        xx += xs[e].x * xs[e].x + xs[e].y * xs[e].y;
-    }
-    const double res = sqrt(block_sum_ac(ss, red, tid));
-    const double xn = sqrt(block_sum_ac(xx, red, tid));
-    const int st = sz_prec_decide(S, res, xn, a.tolsc, a.aiter, a.smax, apprx);
-    if (st == SZ_P_ACTIVE) {
-        __syncthreads();
-        for (int i = tid; i < N; i += AC_NT) {
-            const zd v = rr[(i % 5) * n + i / 5];     // (P r)_i = r_{q(i)}
-            sz::gstore(pb + i, sz::zf{(float)v.x, (float)v.y});
-        }
-    }
-    if (tid == 0) {
-        a.S[s] = S;
-        a.skip[s] = st == SZ_P_ACTIVE ? 0 : 1;
-    }
-    return st;
-}
-
-// One refinement sweep over the systems a.list[0 .. *a.count) (any order):
-// each block takes a contiguous share of the list (whose systems mostly
-// belong to one member, so it restages the profiles rarely), and the
-// systems that continue
-// are appended to a.next (count *a.ncount, cleared by the caller), so that
-// sweeps after convergence cost a handful of blocks.  A block collects its
-// continuing systems in LDS and appends them with one atomic at the end.
-template <bool PROF>
-__global__ __launch_bounds__(AC_NT) __attribute__((amdgpu_waves_per_eu(8)))
-void k_imexop_sweep_listed(const gmember *__restrict__ mem, int nm,
-                           sz_prec_sweep a)
-{
-    constexpr int NPEND = 256;
+    __shared__ int srld[NREF];
     __shared__ int pend[NPEND];               // written by thread 0 only
     __shared__ int npend, pbase;
+    __shared__ int go[MAXSLOT];               // the slot's system continues
     if (threadIdx.x == 0) npend = 0;
+    double *refl = reinterpret_cast<double *>(apmem);
     // uniform values made explicit, so the member's descriptor stays scalar
     const int cnt = __builtin_amdgcn_readfirstlane(*a.count);
     const int per = (cnt + (int)gridDim.x - 1) / (int)gridDim.x;
     const int j0 = (int)blockIdx.x * per, j1 = min(cnt, j0 + per);
     int staged = -1;                          // member whose profiles are in LDS
-    for (int j = j0; j < j1; ++j) {
-        const int s = __builtin_amdgcn_readfirstlane(a.list[j]);
-        const int mi = member_of_sys(mem, nm, s);
-        const gmember &M = mem[mi];
-        const bool stage = mi != staged;
-        staged = mi;
-        __syncthreads();        // the previous system's LDS is read out
-        // the thread index as a value the compiler cannot hold across
-        // systems: what it derives is recomputed per system instead of
-        // occupying registers through the whole loop
+    for (int j = j0, m; j < j1; j += m) {
         int tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));
-        const int st = sweep_body<PROF>(M, s - M.sys0, s, a, tid, stage);
-        if (st == SZ_P_ACTIVE && tid == 0) {
-            if (npend == NPEND) {             // full: flush (more than NPEND
-                const int b = atomicAdd(a.ncount, NPEND);   // systems a block)
-                for (int i = 0; i < NPEND; ++i) a.next[b + i] = pend[i];
-                npend = 0;
-            }
-            pend[npend++] = s;
+        asm volatile("" : "+v"(tid));         // (as in k_imexop_accumulate)
+        const int mi = member_of_sys(mem, nm, __builtin_amdgcn_readfirstlane(a.list[j]));
+        const gmember &M = mem[mi];
+        const bops &w = M.w;
+        const int n = w.n;
+        const int pad = w.max_kl + w.max_ku, fs = n + pad;
+        const size_t ro = (ap_refs(n) + 15) / 16 * 16;
+        int slots = min(min(NTH / n, MAXSLOT), (int)(((size_t)lds - ro) / ap_slot(n, pad)));
+        // even shares of what is left
+        const int rounds = (j1 - j + slots - 1) / slots;
+        slots = (j1 - j + rounds - 1) / rounds;
+        {
+            const int q = tid & 63, sq = q < slots && j + q < j1 ? a.list[j + q] : -1;
+            const unsigned long long in = __ballot(sq >= M.sys0 && sq < M.sys0 + M.nsys);
+            m = in == ~0ull ? 64 : (int)__builtin_ctzll(~in);
         }
+        const int slot = tid / n, r = tid - slot * n;
+        const bool act = slot < m;
+        const int s = act ? a.list[j + slot] : M.sys0, ls = s - M.sys0;
+        zd *al = reinterpret_cast<zd *>(apmem + ro);
+        zd *xs = al + slots * NTERM + w.max_ku;
+        __syncthreads();        // the previous systems' LDS is read out
+        if (staged != mi) {
+            stage_refs<NTH>(M.rf, n, srp, srld, refl);
+            staged = mi;
+        }
+        for (int e = tid; e < m * NTERM; e += NTH) {
+            const int q = e / NTERM, t = e - q * NTERM, lq = a.list[j + q] - M.sys0;
+            al[e] = sz::cmul(M.phi, kappa(M.tab->tk[t], M.km[lq], M.kn[lq]));
+        }
+        const long long o = M.v0 + (long long)ls * 5 * n;
+        zd *x = a.X + o + r;
+        const zd *b = a.B + o + r;
+        sz::zf *pb = a.PB + o + r * 5;
+        double xx = 0, ss = 0;
+        if (act)
+            each<5>([&](auto f_) __attribute__((always_inline)) {
+                constexpr int f = decltype(f_)::value;
+                const sz::zf c = sz::gload(pb + f);   // (P^T c)_e = c_{q^-1(e)}
+                const zd xo = a.first ? zd{0, 0} : sz::gload(x + f * n);
+                const zd v = zd{xo.x + (double)c.x, xo.y + (double)c.y};
+                zd *xf = xs + (slot * 5 + f) * fs;
+                xf[r] = v;
+                ap_margins(w, r, xf);
+                sz::gstore(x + f * n, v);
+                xx += v.x * v.x + v.y * v.y;
+            });
+        __syncthreads();
+        double vx[5], vy[5];
+        if (act) {
+            const int wall = r == 0 ? 0 : (r == n - 1 ? 1 : -1);
+            const zd *xr = xs + slot * 5 * fs + r;
+            double bx[5], by[5];                    // requested before the products
+            each<5>([&](auto f_) __attribute__((always_inline)) {
+                constexpr int f = decltype(f_)::value;
+                const zd v = sz::gload(b + f * n);
+                bx[f] = v.x;
+                by[f] = v.y;
+            });
+            op_rows<true>(w, r, xr - r, al + slot * NTERM, refl, 31u,
+                          [&](auto i_, zd acc, zd mx) __attribute__((always_inline)) {
+                constexpr int i = decltype(i_)::value;
+                zd v;
+                if (i < 4 && wall >= 0 && M.bc.enforce[wall]) {
+                    const zd sc = sz::gload(M.bcs + (size_t)ls * 8 + wall * 4 + i);
+                    const double fac = M.bc.fac[wall][i];
+                    const zd c = zd{xr[i * fs].x - fac * xr[4 * fs].x,
+                                    xr[i * fs].y - fac * xr[4 * fs].y};
+                    const zd p = sz::cmul(sc, c);
+                    v = zd{-p.x, -p.y};
+                } else {
+                    const zd t = zd{acc.x + mx.x, acc.y + mx.y};
+                    v = zd{bx[i] - t.x, by[i] - t.y};
+                }
+                vx[i] = v.x;
+                vy[i] = v.y;
+                ss += v.x * v.x + v.y * v.y;
+            });
+        }
+        __syncthreads();        // x is read out: its place takes the squares
+        double *sq = reinterpret_cast<double *>(xs + (act ? slot : 0) * 5 * fs);
+        if (act) {
+            sq[2 * r] = ss;
+            sq[2 * r + 1] = xx;
+        }
+        __syncthreads();
+        for (int e = tid; e < 2 * G * m; e += NTH) {
+            const int q = e / (2 * G), g = e - q * 2 * G;
+            const double *v = reinterpret_cast<const double *>(xs + q * 5 * fs);
+            double t = 0;
+            for (int i = g; i < 2 * n; i += 2 * G) t += v[i];
+            reinterpret_cast<double *>(al + q * NTERM)[e - q * 2 * G] = t;   // (used up)
+        }
+        __syncthreads();
+        if (tid < m) {
+            double s2 = 0, x2 = 0;
+            const double *part = reinterpret_cast<const double *>(al + tid * NTERM);
+            for (int g = 0; g < G; ++g) {
+                s2 += part[2 * g];
+                x2 += part[2 * g + 1];
+            }
+            const int sy = a.list[j + tid];
+            sz_psys S = a.S[sy];
+            const int st = sz_prec_decide(S, sqrt(s2), sqrt(x2), a.tolsc, a.aiter, a.smax,
+                                          M.apprx[sy - M.sys0]);
+            a.S[sy] = S;
+            a.skip[sy] = st == SZ_P_ACTIVE ? 0 : 1;
+            go[tid] = st == SZ_P_ACTIVE;
+        }
+        __syncthreads();
+        if (act && go[slot])
+            each<5>([&](auto i_) __attribute__((always_inline)) {
+                constexpr int i = decltype(i_)::value;      // (P r)_i = r_{q(i)}
+                sz::gstore(pb + i, sz::zf{(float)vx[i], (float)vy[i]});
+            });
+        if (tid == 0)
+            for (int q = 0; q < m; ++q) {
+                if (!go[q]) continue;
+                if (npend == NPEND) {             // full: flush (more than NPEND
+                    const int p0 = atomicAdd(a.ncount, NPEND);   // systems a block)
+                    for (int i = 0; i < NPEND; ++i) a.next[p0 + i] = pend[i];
+                    npend = 0;
+                }
+                pend[npend++] = a.list[j + q];
+            }
     }
     __syncthreads();
     if (threadIdx.x == 0) pbase = npend ? atomicAdd(a.ncount, npend) : 0;
     __syncthreads();
-    for (int i = threadIdx.x; i < npend; i += AC_NT) a.next[pbase + i] = pend[i];
+    for (int i = threadIdx.x; i < npend; i += NTH) a.next[pbase + i] = pend[i];
 }
 
 // Zero the permuted right hand side entries of the replaced wall equations.
@@ -889,9 +995,32 @@ struct sz_imexop {
     sz_bsplineop *w;
     table host;
     table *dev;
+    double *dc;           // the band coefficients of bops::dc
     int dev_id;
     int ncu;              // compute units of that device
 };
+
+namespace {
+
+bops make_bops(const sz_imexop *op)
+{
+    sz_bsplineop *w = op->w;
+    bops b;
+    b.dt = sz_bsplineop_D_T_device(w);
+    b.dc = op->dc;
+    b.n = sz_bsplineop_n(w);
+    b.ld = sz_bsplineop_ld(w);
+    b.dstride = (long long)b.n * b.ld;
+    b.max_kl = sz_bsplineop_max_kl(w);
+    b.max_ku = sz_bsplineop_max_ku(w);
+    for (int d = 0; d < 3; ++d) {
+        b.kl[d] = sz_bsplineop_kl(w, d);
+        b.ku[d] = sz_bsplineop_ku(w, d);
+    }
+    return b;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -909,13 +1038,38 @@ sz_imexop *sz_imexop_create(const sz_imexop_scenario *s, sz_bsplineop *w,
     op->scen[3] = s->alpha; op->scen[4] = s->gamma;
     op->w = w;
     build_table(op->scen, op->host);
+    if (!shape_ok(op->host)) {
+        delete op;
+        *info = SZ_ERR_LAUNCH;
+        return nullptr;
+    }
     (void)hipGetDevice(&op->dev_id);
     if (hipDeviceGetAttribute(&op->ncu, hipDeviceAttributeMultiprocessorCount,
                               op->dev_id) != hipSuccess || op->ncu < 1)
         op->ncu = 256;
+    const bops b = make_bops(op);
+    const int width = b.max_ku + b.max_kl + 1;
+    std::vector<double> dt(3 * (size_t)b.dstride), dc(3 * (size_t)width * b.n);
     if (hipMalloc(&op->dev, sizeof(table)) != hipSuccess ||
         hipMemcpy(op->dev, &op->host, sizeof(table), hipMemcpyHostToDevice)
+            != hipSuccess ||
+        hipMemcpy(dt.data(), b.dt, dt.size() * sizeof(double), hipMemcpyDeviceToHost)
+            != hipSuccess ||
+        hipMalloc(&op->dc, dc.size() * sizeof(double)) != hipSuccess) {
+        (void)hipFree(op->dev);
+        delete op;
+        *info = SZ_ERR_ALLOC;
+        return nullptr;
+    }
+    for (int d = 0; d < 3; ++d)
+        for (int r = 0; r < b.n; ++r)
+            for (int t = 0; t < width; ++t)
+                dc[((size_t)t * 3 + d) * b.n + r] =
+                    r + t >= b.max_ku && r + t - b.max_ku < b.n
+                        ? dt[d * b.dstride + (size_t)r * b.ld + t] : 0.0;
+    if (hipMemcpy(op->dc, dc.data(), dc.size() * sizeof(double), hipMemcpyHostToDevice)
             != hipSuccess) {
+        (void)hipFree(op->dc);
         (void)hipFree(op->dev);
         delete op;
         *info = SZ_ERR_ALLOC;
@@ -927,6 +1081,7 @@ sz_imexop *sz_imexop_create(const sz_imexop_scenario *s, sz_bsplineop *w,
 void sz_imexop_free(sz_imexop *op)
 {
     if (!op) return;
+    (void)hipFree(op->dc);
     (void)hipFree(op->dev);
     delete op;
 }
@@ -937,28 +1092,38 @@ int sz_imexop_nterms(const sz_imexop *op) { return op ? op->host.nterms : 0; }
 
 namespace {
 
-bops make_bops(sz_bsplineop *w)
-{
-    bops b;
-    b.dt = sz_bsplineop_D_T_device(w);
-    b.n = sz_bsplineop_n(w);
-    b.ld = sz_bsplineop_ld(w);
-    b.dstride = (long long)b.n * b.ld;
-    b.max_kl = sz_bsplineop_max_kl(w);
-    b.max_ku = sz_bsplineop_max_ku(w);
-    for (int d = 0; d < 3; ++d) {
-        b.kl[d] = sz_bsplineop_kl(w, d);
-        b.ku[d] = sz_bsplineop_ku(w, d);
-    }
-    return b;
-}
-
 refs make_refs(const sz_imexop_ref *r, const sz_imexop_refld *ld)
 {
     refs rf;
     std::memcpy(rf.p, r, sizeof(rf.p));
     std::memcpy(rf.ld, ld, sizeof(rf.ld));
     return rf;
+}
+
+// The blocks of an apply launch over systems of n points: the most systems a
+// block of AP_NT threads takes, where two such blocks fit a CU (160 KB of LDS,
+// 6 KB of it left to the kernels' own in each), else a block of AP_NT1.
+struct apply_shape {
+    int nt, slots, per_cu;
+};
+size_t ap_bytes(int n, int pad, int slots)
+{
+    return (ap_refs(n) + 15) / 16 * 16 + slots * ap_slot(n, pad);
+}
+constexpr size_t AP_LDS2 = 74 * 1024, AP_LDS1 = 150 * 1024;
+constexpr int AP_PAD = 16;     // of the refined solve's band shapes (k <= 8), and more
+// (Two blocks of three waves a SIMD hide each other's loads; for the larger n
+// one block of twice the threads keeps as many waves.)
+apply_shape apply_blocks(int n, int pad)
+{
+    if (n <= AP_NT && ap_bytes(n, pad, 1) <= AP_LDS2) {
+        int slots = std::min(AP_NT / n, 64);
+        while (ap_bytes(n, pad, slots) > AP_LDS2) --slots;
+        return {AP_NT, slots, 2};
+    }
+    int slots = std::max(1, AP_NT1 / n);
+    while (slots > 1 && ap_bytes(n, pad, slots) > AP_LDS1) --slots;
+    return {AP_NT1, slots, 1};
 }
 
 // Positions of (rho E, rho u, rho v, rho w, rho); returns S or a negative
@@ -1001,7 +1166,7 @@ int sz_rholut_imexop_packc_batched(
     int field_of[5];
     const int S = positions(pos, field_of);
     if (S <= 0) return S == 0 ? -7 : -6 + S;
-    const bops w = make_bops(op->w);
+    const bops w = make_bops(op);
     const sz_bsmbsm g = sz_bsmbsm_construct(S, w.n, w.max_kl, w.max_ku);
     if (A_T) *A_T = g;
     if (ldpatpt < g.LD) return -14;
@@ -1109,32 +1274,38 @@ int sz_internal_imexop_accumulate_masked(
         if ((in[f] == nullptr) != (out[f] == nullptr)) return -7;
     if (nsys < 0) return -14;
     if (nsys == 0) return 0;
-    const bops w = make_bops(op->w);
-    size_t lds = sizeof(zd) * (MAXTERMS + 20 * (size_t)w.n);
-    if (lds > 156 * 1024) return SZ_ERR_LDS;   // 160 KB less the staged tables
-    // blocks resident per CU (two at most: 1024 threads each), with the
-    // kernel's static LDS and 1 KB allocation granules; the profiles are
-    // staged whenever they fit: a persistent block stages them once for all
-    // of its systems, which costs less than gathering them per term even
-    // where it leaves one block per CU instead of two
-    auto per_cu = [](size_t b) {
-        const size_t a = (b + 2048 + 1023) / 1024 * 1024;
-        return (int)std::min<size_t>(2, 160 * 1024 / a);
-    };
-    const bool staged = lds + REFL_BYTES(w.n) <= 156 * 1024;
-    if (staged) lds += REFL_BYTES(w.n);
-    // persistent blocks: as many as stay resident, each taking every
-    // grid-th system
-    const int grid = (int)std::min<long long>(nsys, (long long)op->ncu * per_cu(lds));
+    const bops w = make_bops(op);
+    if (sizeof(zd) * (MAXTERMS + 20 * (size_t)w.n) > 156 * 1024) return SZ_ERR_LDS;
+    const int pad = w.max_kl + w.max_ku;
+    const apply_shape sh = apply_blocks(w.n, pad);
+    if (ap_bytes(w.n, pad, 1) > 158 * 1024) return SZ_ERR_LDS;
+    // persistent blocks: as many as stay resident, with even shares
+    const long long nblk = (long long)op->ncu * sh.per_cu;
+    const long long rounds = (nsys + nblk * sh.slots - 1) / (nblk * sh.slots);
+    const int slots = (int)((nsys + nblk * rounds - 1) / (nblk * rounds));
+    const int grid = (int)std::min<long long>((nsys + slots - 1) / slots, nblk);
     const int bz = beta[0] == 0 && beta[1] == 0;
-    hipLaunchKernelGGL((staged ? k_imexop_accumulate<true> : k_imexop_accumulate<false>),
-                       dim3(grid), dim3(AC_NT), lds,
-                       (hipStream_t)stream, op->dev, w, make_refs(r, ld),
-                       zd{phi[0], phi[1]}, km, kn, (const zd *)in[0],
-                       (const zd *)in[1], (const zd *)in[2], (const zd *)in[3],
-                       (const zd *)in[4], inoff, instride, zd{beta[0], beta[1]},
-                       bz, (zd *)out[0], (zd *)out[1], (zd *)out[2],
-                       (zd *)out[3], (zd *)out[4], outoff, outstride, skip, nsys);
+    fields F;
+    bool all = true;
+    for (int f = 0; f < 5; ++f) {
+        F.in[f] = (const zd *)in[f];
+        F.out[f] = (zd *)out[f];
+        all = all && in[f];
+    }
+#define SZ_ACC(ALL_, NT_)                                                             \
+    hipLaunchKernelGGL((k_imexop_accumulate<ALL_, NT_>), dim3(grid), dim3(NT_),       \
+                       ap_bytes(w.n, pad, slots), (hipStream_t)stream, op->dev, w,         \
+                       make_refs(r, ld), zd{phi[0], phi[1]}, km, kn, F, inoff,        \
+                       instride, zd{beta[0], beta[1]}, bz, outoff, outstride, skip,   \
+                       nsys, slots)
+    if (sh.nt == AP_NT) {
+        if (all) SZ_ACC(true, AP_NT);
+        else SZ_ACC(false, AP_NT);
+    } else {
+        if (all) SZ_ACC(true, AP_NT1);
+        else SZ_ACC(false, AP_NT1);
+    }
+#undef SZ_ACC
     return launch_ok() ? 0 : SZ_ERR_LAUNCH;
 }
 
@@ -1158,7 +1329,7 @@ int sz_internal_imexop_pack32(const sz_imexop *op, const double *phi,
                               void *bcs, double *frob, void *stream)
 {
     if (!op || !phi || !km || !kn || !r || !ld || !bc) return -1;
-    const bops w = make_bops(op->w);
+    const bops w = make_bops(op);
     const sz_bsmbsm g = sz_bsmbsm_construct(5, w.n, w.max_kl, w.max_ku);
     if (ldlu < g.LD + g.KL) return -9;
     if (nsys < 0) return -11;
@@ -1205,7 +1376,7 @@ int sz_internal_imexop_member(const sz_imexop *op, const double *phi,
     if (!op || !phi || !r || !ld || !bc || !out) return -1;
     gmember m{};
     m.tab = op->dev;
-    m.w = make_bops(op->w);
+    m.w = make_bops(op);
     if (!m.w.dt) return SZ_ERR_ALLOC;
     m.rf = make_refs(r, ld);
     m.phi = zd{phi[0], phi[1]};
@@ -1250,69 +1421,40 @@ int sz_internal_imexop_pack_listed(const void *dmem, int nm, int nsys, int ldmax
     return launch_ok() ? 0 : SZ_ERR_LAUNCH;
 }
 
-// LDS of a sweep block for systems of up to n coefficients per field.
-// LDS of a sweep block for systems of up to n points, with (prof) or
-// without the reference profiles.
-static size_t sweep_lds(int n, bool prof = true)
-{
-    return sizeof(zd) * (MAXTERMS + 25 * (size_t)n) + (prof ? REFL_BYTES(n) : 0);
-}
-
-// Sweep blocks resident per CU (two at most: 1,024 threads each) for systems
-// of up to n points, with or without the profiles (160 KB of LDS, 1 KB
-// granules, the kernel's static LDS included).
-static int sweep_per_cu(int n, bool prof)
-{
-    const size_t stat = 3072;           // static LDS of the sweep, rounded up
-    const size_t a = (sweep_lds(n, prof) + stat + 1023) / 1024 * 1024;
-    return (int)std::min<size_t>(2, 160 * 1024 / a);
-}
-
-// Whether the sweep of systems of up to nmax points stages the members'
-// profiles: where two blocks per CU still fit with them, or where even
-// without them only one does.
-static bool sweep_prof(int nmax)
-{
-    return sweep_per_cu(nmax, true) == 2 || sweep_per_cu(nmax, false) < 2;
-}
-
-// The sweep's tier bounds: the largest n whose blocks fit two to a CU with
-// the profiles staged (which = 0) and with them gathered (which = 1).  Each
-// tier runs a launch of its own, so that the larger systems do not size the
-// LDS of every block.
+// The sweep's tier bounds: the largest n of which two blocks fit a CU
+// (which = 0) and the largest of which a block of AP_NT1 threads holds two
+// systems (which = 1).  Each tier runs a launch of its own, so that the larger
+// systems do not size the LDS of every block.
 int sz_internal_imexop_sweep_tier_n(int which)
 {
     int n = 1;
-    while (sweep_per_cu(n + 1, which == 0) == 2) ++n;
+    while (which == 0 ? apply_blocks(n + 1, AP_PAD).nt == AP_NT : n + 1 <= AP_NT1 / 2) ++n;
     return n;
 }
 
 // One refinement sweep of the mixed precision solve over the listed systems
-// (a->list, *a->count <= nsys; nmax the largest n among them): a grid of at
-// most 1024 blocks strides over the list.
+// (a->list, *a->count <= nsys; nmax the largest n among them): as many blocks
+// as stay resident, each with one contiguous share of the list.
 int sz_internal_imexop_sweep_listed(const void *dmem, int nm, int nsys,
                                     int nmax, const sz_prec_sweep *a,
                                     void *stream)
 {
     if (nsys <= 0) return 0;
-    // the member's profiles staged in LDS where that keeps two blocks per
-    // CU, or where one is all that fits anyway (and they fit), else
-    // gathered per term
-    const bool prof = sweep_prof(nmax) && sweep_per_cu(nmax, true) >= 1;
-    const size_t lds = sweep_lds(nmax, prof);
-    if (lds > 156 * 1024) return SZ_ERR_LDS;
-    // as many blocks as stay resident, each with one contiguous share of the
-    // list (fewer member changes, so fewer restagings of the profiles)
+    if (sizeof(zd) * (MAXTERMS + 25 * (size_t)nmax) > 156 * 1024) return SZ_ERR_LDS;
+    const apply_shape sh = apply_blocks(nmax, AP_PAD);
+    const size_t lds = sh.nt == AP_NT ? AP_LDS2 : AP_LDS1;
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) !=
             hipSuccess || ncu < 1)
         ncu = 256;
-    const int grid = (int)std::min<long long>(
-        nsys, (long long)ncu * std::max(1, sweep_per_cu(nmax, prof)));
-    hipLaunchKernelGGL((prof ? k_imexop_sweep_listed<true> : k_imexop_sweep_listed<false>),
-                       dim3(grid), dim3(AC_NT), lds,
-                       (hipStream_t)stream, (const gmember *)dmem, nm, *a);
+    const int grid = (int)std::min<long long>(nsys, (long long)ncu * sh.per_cu);
+    if (sh.nt == AP_NT)
+        hipLaunchKernelGGL(k_imexop_sweep_listed<AP_NT>, dim3(grid), dim3(AP_NT), lds,
+                           (hipStream_t)stream, (const gmember *)dmem, nm, *a, (int)lds);
+    else
+        hipLaunchKernelGGL(k_imexop_sweep_listed<AP_NT1>, dim3(grid), dim3(AP_NT1), lds,
+                           (hipStream_t)stream, (const gmember *)dmem, nm, *a, (int)lds);
     return launch_ok() ? 0 : SZ_ERR_LAUNCH;
 }
 
