@@ -31,6 +31,8 @@
 #include <string>
 #include <vector>
 
+extern "C" const double *sz_internal_bsplineop_D_C_device(sz_bsplineop *w);
+
 namespace {
 
 using sz::zd;
@@ -133,7 +135,7 @@ struct deriv_args {
     const zd *s;
     zd *vals, *auxw;
     long long F;
-    const double *dt;            // D_T of derivatives 0, 1, 2, each n * ld
+    const double *dc;            // derivatives 0, 1, 2 by band offset, each ld * n
     int n, ld, kuaddr;
     int kl0, ku0, kl1, ku1, kl2, ku2;
     int xkeep, zabs, Xw, dNz, pb;
@@ -149,20 +151,6 @@ __device__ inline double pow_int(double x, int n)
         x *= x;
     } while (n);
     return v;
-}
-
-__device__ inline zd band_apply(const double *col, const zd *xp, int i, int n,
-                                int kl, int ku)
-{
-    const int j0 = max(0, i - ku), j1 = min(n - 1, i + kl);
-    zd acc = {0, 0};
-    for (int j = j0; j <= j1; ++j) {
-        const double d = col[j];
-        const zd xv = xp[j];
-        acc.x = fma(d, xv.x, acc.x);
-        acc.y = fma(d, xv.y, acc.y);
-    }
-    return acc;
 }
 
 // (i kx)^DX (i kz)^DZ x, and the same plus 1 * y
@@ -186,6 +174,13 @@ __device__ inline zd dwave_acc(zd x, zd y, int mf, int nf, double tpx, double tp
     return sz::cadd_rn(dwave<DX, DZ>(x, mf, nf, tpx, tpz), by);
 }
 
+// A field's collocation values and derivatives on the retained pencils, pb of
+// them a block.  Bound by the bytes written (10 arrays a field).  The pencils
+// wait in LDS with zeros around them, for the columns a row's band has outside
+// the matrix; the coefficients come by band offset, 512 contiguous bytes a
+// wavefront (each lane its own row's run touched 64 cache lines a load, which
+// bound the kernel: 1.59 ms for 18,336 pencils of n = 192, now 0.84 ms, 3.4
+// TB/s; n = 96, 4,560 pencils: 101 -> 87 us).
 __global__ __launch_bounds__(NT)
 void k_derivs(deriv_args a)
 {
@@ -205,10 +200,12 @@ void k_derivs(deriv_args a)
         return ((long long)(wz < 0 ? wz + a.dNz : wz) * a.Xw + x) * n;
     };
     const zd *sf = a.s + (size_t)f * F;
-    for (int e = threadIdx.x; e < np * n; e += blockDim.x) {
-        const int lp = e / n, i = e - lp * n;
+    const int ps = n + a.ld - 1;                 // kuaddr zeros, n values, zeros
+    for (int e = threadIdx.x; e < np * ps; e += blockDim.x) {
+        const int lp = e / ps, i = e - lp * ps - a.kuaddr;
         int x, wz;
-        pen[e] = sf[offset(q0 + lp, x, wz) + i];
+        const long long o = offset(q0 + lp, x, wz);
+        pen[e] = i >= 0 && i < n ? sz::gload(sf + o + i) : zd{0, 0};
     }
     __syncthreads();
     const zd one = {1.0, 0.0};
@@ -216,12 +213,31 @@ void k_derivs(deriv_args a)
         const int lp = e / n, i = e - lp * n;
         int x, wz;
         const long long o = offset(q0 + lp, x, wz) + i;
-        const zd *xp = pen + lp * n;
-        const double *col = a.dt + (size_t)i * a.ld + a.kuaddr - i;
+        const zd *xp = pen + lp * ps + i;
+        const double *col = a.dc;
         const size_t dstep = (size_t)n * a.ld;
-        const zd v = sz::cmul(one, band_apply(col, xp, i, n, a.kl0, a.ku0));
-        const zd y = sz::cmul(one, band_apply(col + dstep, xp, i, n, a.kl1, a.ku1));
-        const zd yy = sz::cmul(one, band_apply(col + 2 * dstep, xp, i, n, a.kl2, a.ku2));
+        zd s0{0, 0}, s1{0, 0}, s2{0, 0};
+#pragma unroll 4
+        for (int t = 0; t < a.ld; ++t, col += n) {
+            const double d0 = sz::gmem(col)[(unsigned)i];
+            const double d1 = sz::gmem(col + dstep)[(unsigned)i];
+            const double d2 = sz::gmem(col + 2 * dstep)[(unsigned)i];
+            const zd xv = xp[t];
+            const int j = t - a.kuaddr;
+            if (j >= -a.ku0 && j <= a.kl0) {
+                s0.x = fma(d0, xv.x, s0.x);
+                s0.y = fma(d0, xv.y, s0.y);
+            }
+            if (j >= -a.ku1 && j <= a.kl1) {
+                s1.x = fma(d1, xv.x, s1.x);
+                s1.y = fma(d1, xv.y, s1.y);
+            }
+            if (j >= -a.ku2 && j <= a.kl2) {
+                s2.x = fma(d2, xv.x, s2.x);
+                s2.y = fma(d2, xv.y, s2.y);
+            }
+        }
+        const zd v = sz::cmul(one, s0), y = sz::cmul(one, s1), yy = sz::cmul(one, s2);
         const double tx = a.tpx, tz = a.tpz;
         a.vals[f * F + o] = v;
         if (f == 0) {
@@ -709,8 +725,8 @@ int sz_channel_nonlinear_time(sz_channel *h, int which, int zeroth, double time,
         a.vals = h->vals;
         a.auxw = h->auxw;
         a.F = F;
-        a.dt = sz_bsplineop_D_T_device(h->bop);
-        if (!a.dt) return SZ_ERR_ALLOC;
+        a.dc = sz_internal_bsplineop_D_C_device(h->bop);
+        if (!a.dc) return SZ_ERR_ALLOC;
         a.n = sz_bsplineop_n(h->bop);
         if (a.n != n) return -3;
         a.ld = sz_bsplineop_ld(h->bop);
@@ -732,7 +748,7 @@ int sz_channel_nonlinear_time(sz_channel *h, int which, int zeroth, double time,
         a.tpz = twopi / sp.Lz;
         const int nthr = (int)std::min<long long>(NT, ((long long)pb * n + 63) / 64 * 64);
         hipLaunchKernelGGL(k_derivs, dim3((unsigned)((h->nsys + pb - 1) / pb), 5),
-                           dim3(nthr), (size_t)pb * n * sizeof(zd), st, a);
+                           dim3(nthr), (size_t)pb * (n + a.ld - 1) * sizeof(zd), st, a);
         if (!ok()) return SZ_ERR_LAUNCH;
     }
     if (!fused) rc = h->zero_dealias(s, 5);

@@ -269,7 +269,7 @@ __device__ inline zd weight_staged(const int *gt0, const int *gnt, const int *tr
 
 struct bops {
     const double *dt;     // derivative d's transposed band at dt + d * dstride
-    const double *dc;     // its rows' element t (from 0) for every row: dc[(3 t + d) n + r]
+    const double *dc;     // the same by band offset: dc[d * dstride + t * n + r]
     long long dstride;
     int n, ld, max_kl, max_ku;
     int kl[3], ku[3];
@@ -342,10 +342,10 @@ __device__ __forceinline__ void op_rows(const bops &w, int r, const zd *xs, cons
         dx[decltype(k_)::value] = dy[decltype(k_)::value] = 0;
     });
     auto fetch = [&](int t, double (&a)[3]) __attribute__((always_inline)) {
-        const double *p = w.dc + (long long)(min(t, hi) + w.max_ku) * 3 * n;
+        const double *p = w.dc + (long long)(min(t, hi) + w.max_ku) * n;
         each<3>([&](auto o_) __attribute__((always_inline)) {
             constexpr int op = decltype(o_)::value;
-            a[op] = sz::gmem(p + op * n)[(unsigned)r];
+            a[op] = sz::gmem(p + op * w.dstride)[(unsigned)r];
         });
     };
     auto products = [&](auto full) __attribute__((always_inline)) {
@@ -990,12 +990,13 @@ inline bool launch_ok() { return hipGetLastError() == hipSuccess; }
 
 }  // namespace
 
+extern "C" const double *sz_internal_bsplineop_D_C_device(sz_bsplineop *w);
+
 struct sz_imexop {
     double scen[5];
     sz_bsplineop *w;
     table host;
     table *dev;
-    double *dc;           // the band coefficients of bops::dc
     int dev_id;
     int ncu;              // compute units of that device
 };
@@ -1007,7 +1008,7 @@ bops make_bops(const sz_imexop *op)
     sz_bsplineop *w = op->w;
     bops b;
     b.dt = sz_bsplineop_D_T_device(w);
-    b.dc = op->dc;
+    b.dc = sz_internal_bsplineop_D_C_device(w);
     b.n = sz_bsplineop_n(w);
     b.ld = sz_bsplineop_ld(w);
     b.dstride = (long long)b.n * b.ld;
@@ -1047,29 +1048,9 @@ sz_imexop *sz_imexop_create(const sz_imexop_scenario *s, sz_bsplineop *w,
     if (hipDeviceGetAttribute(&op->ncu, hipDeviceAttributeMultiprocessorCount,
                               op->dev_id) != hipSuccess || op->ncu < 1)
         op->ncu = 256;
-    const bops b = make_bops(op);
-    const int width = b.max_ku + b.max_kl + 1;
-    std::vector<double> dt(3 * (size_t)b.dstride), dc(3 * (size_t)width * b.n);
     if (hipMalloc(&op->dev, sizeof(table)) != hipSuccess ||
         hipMemcpy(op->dev, &op->host, sizeof(table), hipMemcpyHostToDevice)
-            != hipSuccess ||
-        hipMemcpy(dt.data(), b.dt, dt.size() * sizeof(double), hipMemcpyDeviceToHost)
-            != hipSuccess ||
-        hipMalloc(&op->dc, dc.size() * sizeof(double)) != hipSuccess) {
-        (void)hipFree(op->dev);
-        delete op;
-        *info = SZ_ERR_ALLOC;
-        return nullptr;
-    }
-    for (int d = 0; d < 3; ++d)
-        for (int r = 0; r < b.n; ++r)
-            for (int t = 0; t < width; ++t)
-                dc[((size_t)t * 3 + d) * b.n + r] =
-                    r + t >= b.max_ku && r + t - b.max_ku < b.n
-                        ? dt[d * b.dstride + (size_t)r * b.ld + t] : 0.0;
-    if (hipMemcpy(op->dc, dc.data(), dc.size() * sizeof(double), hipMemcpyHostToDevice)
             != hipSuccess) {
-        (void)hipFree(op->dc);
         (void)hipFree(op->dev);
         delete op;
         *info = SZ_ERR_ALLOC;
@@ -1081,7 +1062,6 @@ sz_imexop *sz_imexop_create(const sz_imexop_scenario *s, sz_bsplineop *w,
 void sz_imexop_free(sz_imexop *op)
 {
     if (!op) return;
-    (void)hipFree(op->dc);
     (void)hipFree(op->dev);
     delete op;
 }
