@@ -114,6 +114,18 @@ __device__ inline cpx<R> wave_csum(cpx<R> v)
     return cpx<R>{wave_sum_asc(v.x), wave_sum_asc(v.y)};
 }
 
+// The largest of the 64 lanes' values (no NaN among them).
+template <typename R>
+__device__ __forceinline__ R wave_max(R v)
+{
+    v = fmax(v, dpp_r<0xB1>(v));            // the stages of wave_sum_asc
+    v = fmax(v, dpp_r<0x4E>(v));
+    v = fmax(v, dpp_r<0x141>(v));
+    v = fmax(v, dpp_r<0x140>(v));
+    return fmax(fmax(readlane_r(v, 0), readlane_r(v, 16)),
+                fmax(readlane_r(v, 32), readlane_r(v, 48)));
+}
+
 constexpr int TRF_PF = 8;   // incoming rows prefetched ahead of their step
 
 template <typename R>
@@ -197,13 +209,28 @@ void k_gbtrf(int n, int kl, int ku, cpx<R> *__restrict__ ab, int ldab,
                 // NaN never beats a number, a NaN in the first slot wins)
                 R best = R(-1);
                 int bidx = 0x7fffffff;
-                for (int r = tid; r <= km; r += 64) {
-                    int rs = rs0 + r; if (rs >= WR) rs -= WR;
-                    R a = sz::cabs1(W[rs * WC + cs0]);
-                    if (a != a) a = R(-1);
-                    if (a > best || (a == best && r < bidx)) { best = a; bidx = r; }
+                if (kl < 64) {
+                    // a row a lane: the maximum by DPP, then its first lane.
+                    // (Value and index through six lane exchanges, as for more
+                    // rows: 600 systems n = 301, kl 17, ku 11 in 763 us, so
+                    // 595.)
+                    R a = R(-2);
+                    if (tid <= km) {
+                        int rs = rs0 + tid; if (rs >= WR) rs -= WR;
+                        a = sz::cabs1(W[rs * WC + cs0]);
+                        if (a != a) a = R(-1);
+                    }
+                    best = wave_max(a);
+                    bidx = (int)__builtin_ctzll(__ballot(a == best));
+                } else {
+                    for (int r = tid; r <= km; r += 64) {
+                        int rs = rs0 + r; if (rs >= WR) rs -= WR;
+                        R a = sz::cabs1(W[rs * WC + cs0]);
+                        if (a != a) a = R(-1);
+                        if (a > best || (a == best && r < bidx)) { best = a; bidx = r; }
+                    }
+                    argmax_cabs1(best, bidx);
                 }
-                argmax_cabs1(best, bidx);
                 const T a0 = W[rs0 * WC + cs0];
                 const R a0abs = sz::cabs1(a0);
                 const int p = (a0abs != a0abs) ? 0 : bidx;
