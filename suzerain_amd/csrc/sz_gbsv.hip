@@ -1676,7 +1676,7 @@ void k_gbtrf_panel(int n, cpx<R> *__restrict__ ab, int ldab, long long sab,
     static_assert(kl >= NB && ku >= NB, "interchanges reach every panel column");
     static_assert(NT == 0 || NT == 2 * NB, "tail");
     __shared__ T pbuf[NB * PS];
-    __shared__ T qbuf[(NB + 2) * 64];              // what the next block needs
+    __shared__ alignas(16) T qbuf[(NB + 2) * 64];  // what the next block needs
     __shared__ T tail[NT > 0 ? NT * PR : 1];
     __shared__ T tailb[NT > 0 ? NT : 1];
 
@@ -2163,12 +2163,19 @@ void k_gbtrf_panel(int n, cpx<R> *__restrict__ ab, int ldab, long long sab,
 
 // Launches k_gbtrf_panel for the band shapes it is instantiated for -- kl =
 // ku = 34 (five interleaved fields, k = 8 operators), kl = ku = 24 (k = 6)
-// and kl = 34, ku = 20 -- and returns whether the shape is one of them.
+// and kl = 34, ku = 20 -- and returns whether the call is one for it.  Its
+// transfers to LDS move a complex double as 16 bytes, which are not documented
+// for less than 16-byte alignment; an array aligned as C's double complex (8
+// bytes) goes to the kernels whose loads the compiler chose.  (A grouped
+// launch's arrays are the library's own.)
 template <typename R, bool UT>
 bool launch_panel(int n, int kl, int ku, void *ab, int ldab, long long sab, int *ipiv,
                   long long sipiv, int *info, const int *skip, int nsys, void *b,
                   long long sb, const sz::gsys *gs, hipStream_t stream)
 {
+    if (sizeof(R) == 8 && !gs &&
+        (reinterpret_cast<uintptr_t>(ab) | reinterpret_cast<uintptr_t>(b)) % 16 != 0)
+        return false;
 #define SZ_PANEL(WR_, KV_)                                                      \
     hipLaunchKernelGGL((k_gbtrf_panel<R, WR_, KV_, UT, panel_waves(sizeof(R), WR_, UT)>), \
                        dim3(nsys), dim3(64), 0, stream, n,                      \
@@ -2183,7 +2190,7 @@ bool launch_panel(int n, int kl, int ku, void *ab, int ldab, long long sab, int 
 }
 
 // Factorization kernels: k_gbtrf_panel for the channel band shapes and the
-// LDS window kernel k_gbtrf for every other shape.  SZ_GBTRF_KERNEL = "lds"
+// LDS window kernel k_gbtrf for every other call.  SZ_GBTRF_KERNEL = "lds"
 // (or "lds64"/"lds128", fewer threads) forces the LDS kernel.
 template <typename R>
 int launch_gbtrf(int n, int kl, int ku, void *ab, int ldab, long long sab,
@@ -2228,7 +2235,8 @@ int launch_gbtrf(int n, int kl, int ku, void *ab, int ldab, long long sab,
 
 // Factorization fused with the U^T half of a transposed solve of one right
 // hand side per system (b, stride sb, overwritten by y); returns 1 when the
-// band shape has no fused kernel (the caller then factors and solves apart).
+// band shape or the arrays' alignment has no fused kernel (the caller then
+// factors and solves apart).
 template <typename R>
 int launch_gbtrf_ut(int n, int kl, int ku, void *ab, int ldab, long long sab,
                     int *ipiv, long long sipiv, int *info, void *b, long long sb,

@@ -88,3 +88,56 @@ def test_infinities_and_zero_columns(gpu, kl, ku):
     ab[4, 70, kl + ku] = 5e-324              # 1/pivot overflows
     ab[4, 70, kl + ku + 1:] = 0.0
     _check(gpu, ab, kl, ku, "z")
+
+
+@pytest.mark.parametrize("kl,ku", SHAPES)
+def test_arrays_aligned_as_c_double_complex(gpu, kl, ku):
+    """Band storage and right hand sides 8 bytes off a 16-byte boundary, which
+    C's double complex allows: the panel kernel's 16-byte transfers to LDS are
+    not for them.  The factorization still gives the oracle's bits; the fused
+    one declines, and has written nothing."""
+    import ctypes as C
+    import torch
+    from suzerain_amd._lib import load
+    lib = load()
+    i32, i64, vp = C.c_int, C.c_longlong, C.c_void_p
+    f_ut = lib.sz_internal_zgbtrf_ut
+    f_ut.restype = i32
+    f_ut.argtypes = [i32, i32, i32, vp, i32, i64, vp, i64, vp, vp, i64, i32, vp]
+    rng = np.random.default_rng(kl + 2 * ku)
+    N, nb, ldab = 77, 2, 2 * kl + ku + 1
+    ab = _bands(rng, nb, N, kl, ku, 0.0)
+    b = rng.standard_normal((nb, N)) + 1j * rng.standard_normal((nb, N))
+
+    def device(a, off):                      # a's doubles from element `off` on
+        flat = a.reshape(-1).view(np.float64)
+        d = torch.zeros(flat.size + 2, dtype=torch.float64, device=gpu)
+        assert d.data_ptr() % 16 == 0
+        d[off:off + flat.size] = torch.from_numpy(flat).to(gpu)
+        return d, d.data_ptr() + 8 * off
+
+    def host(d, off, a):
+        return d[off:off + 2 * a.size].cpu().numpy().view(np.complex128).reshape(a.shape)
+
+    stream = vp(torch.cuda.current_stream().cuda_stream)
+    ipiv = torch.zeros((nb, N), dtype=torch.int32, device=gpu)
+    info = torch.zeros((nb,), dtype=torch.int32, device=gpu)
+    for oa, ob in ((1, 0), (0, 1)):
+        ad, ap = device(ab, oa)
+        bd, bp = device(b, ob)
+        assert f_ut(N, kl, ku, ap, ldab, ldab * N, ipiv.data_ptr(), N, info.data_ptr(),
+                    bp, N, nb, stream) == 1
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(host(ad, oa, ab), ab)
+        np.testing.assert_array_equal(host(bd, ob, b), b)
+    ad, ap = device(ab, 1)
+    assert lib.sz_zgbtrf_batched(N, kl, ku, ap, ldab, ldab * N, ipiv.data_ptr(), N,
+                                 info.data_ptr(), nb, stream) == 0
+    torch.cuda.synchronize()
+    lu = host(ad, 1, ab)
+    for s in range(nb):
+        ref = ab[s].reshape(-1).copy()
+        rinfo, rpiv = oracle.zgbtrf(N, kl, ku, ref, ldab)
+        assert int(info[s]) == rinfo == 0
+        np.testing.assert_array_equal(ipiv[s].cpu().numpy(), rpiv)
+        np.testing.assert_array_equal(lu[s], ref.reshape(N, ldab))
