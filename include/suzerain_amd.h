@@ -573,8 +573,8 @@ typedef struct sz_ensemble_opts {
     int nstreams;         /* explicit-stage streams (1..max_streams)        */
     int max_streams;      /* streams (and scratch sets) created, <= 8       */
     int graph;            /* capture steps in a hipGraph                    */
-    int lu_bs;            /* factorization unroll, 4 or 8 (0: 8): accepted,
-                             one kernel serves both                         */
+    int lu_bs;            /* factorization unroll, 4 or 8 (0: 8): kept and
+                             reported, selects nothing (one kernel)         */
 } sz_ensemble_opts;
 sz_ensemble *sz_ensemble_create(int nmembers, const sz_channel_spec *specs,
                                 const double *dt, const sz_ensemble_opts *opts,
@@ -601,10 +601,11 @@ int sz_ensemble_check(sz_ensemble *e);
 /* Per-system outcome of the last solve (sz_channel_solver_stats codes),
  * members' systems in the solver's order. */
 void *sz_ensemble_solver_stats(sz_ensemble *e, int which);
-/* Autotune the explicit-stage stream count and the factorization unroll by
- * timing `steps` eager steps per candidate from the same saved states; the
- * states are restored afterwards; a captured step is dropped and captured
- * again at the next step. */
+/* Autotune the explicit-stage stream count by timing `steps` eager steps per
+ * candidate (1 to 4 streams, at most max_streams) from the same saved states;
+ * the states are restored afterwards; a captured step is dropped and captured
+ * again at the next step.  sz_ensemble_tuning: the choice, the option lu_bs (8
+ * after tuning where it was 0) and a time per candidate, in order. */
 int sz_ensemble_autotune(sz_ensemble *e, int steps);
 int sz_ensemble_tuning(const sz_ensemble *e, int *nstreams, int *lu_bs,
                        double *trial_ms, int max, int *ntrials);

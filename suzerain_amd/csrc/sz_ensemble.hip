@@ -71,7 +71,7 @@ struct sz_ensemble {
     hipGraphExec_t exec = nullptr;
     double tuned_ms = 0;
     std::vector<double> trial_ms;         // autotune: per candidate
-    int lu_bs = 0;                        // option as given: one kernel serves all
+    int lu_bs = 0;                        // option as given; selects nothing
     long long bytes = 0;
     std::vector<void *> owned;
 
@@ -491,10 +491,10 @@ void *sz_ensemble_solver_stats(sz_ensemble *e, int which)
     return e ? sz_prec_stats(e->prec, which) : nullptr;
 }
 
-// The autotuner: every candidate mapping -- explicit-stage streams 1, 2, 4
-// (members dealt round-robin) x factorization unroll 4 or 8 steps -- timed
-// over `steps` eager steps after a warm step, from the same saved states,
-// factors refactored for each; the fastest is kept and the states restored.
+// The autotuner: every candidate mapping -- 1 to 4 explicit-stage streams
+// (members dealt round-robin) -- timed over `steps` eager steps after a warm
+// step, from the same saved states, factors refactored for each; the fastest is
+// kept and the states restored.
 int sz_ensemble_autotune(sz_ensemble *e, int steps)
 {
     if (!e) return -1;
@@ -527,27 +527,23 @@ int sz_ensemble_autotune(sz_ensemble *e, int steps)
     e->graph = 0;                      // trials run eagerly
     sz_prec_set_graph(e->prec, 0);
     double best = -1;
-    int best_ns = e->nstreams, best_bs = e->lu_bs ? e->lu_bs : 8;
+    int best_ns = e->nstreams;
     e->trial_ms.clear();
     const int cand_ns[4] = {1, 2, 3, 4};
-    const int cand_bs[2] = {4, 8};     // one kernel: each stream count is timed twice
     for (int a = 0; a < 4 && !rc; ++a) {
         if (cand_ns[a] > e->maxstreams) continue;
-        for (int b = 0; b < 2 && !rc; ++b) {
-            restore();
-            e->assign_streams(cand_ns[a]);
-            const double ms = e->trial(steps);
-            e->trial_ms.push_back(ms);
-            if (ms > 0 && (best < 0 || ms < best)) {
-                best = ms;
-                best_ns = cand_ns[a];
-                best_bs = cand_bs[b];
-            }
+        restore();
+        e->assign_streams(cand_ns[a]);
+        const double ms = e->trial(steps);
+        e->trial_ms.push_back(ms);
+        if (ms > 0 && (best < 0 || ms < best)) {
+            best = ms;
+            best_ns = cand_ns[a];
         }
     }
     restore();
     e->assign_streams(best_ns);
-    e->lu_bs = best_bs;
+    if (!e->lu_bs) e->lu_bs = 8;       // what the option's 0 stands for
     e->graph = graph;
     sz_prec_set_graph(e->prec, graph);
     e->tuned_ms = best;

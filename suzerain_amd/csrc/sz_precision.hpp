@@ -151,5 +151,5 @@ void sz_prec_counts(const sz_prec *h, int *factored, int *restarted,
                     int *fallback);
 // Total systems over all members.
 int sz_prec_nsys(const sz_prec *h);
-// Factorization unroll (autotuner) and graph mode switches.
+// Graph mode switch.
 void sz_prec_set_graph(sz_prec *h, int graph);

@@ -100,14 +100,16 @@ def test_autotune_leaves_states(gpu):
     W = [_initial(c, gpu) for c in members]
     dts = [2e-3, 1.5e-3, 2.5e-3, 1e-3]
     a = Ensemble(members, dt=dts, solver=SPEC, graph=True, max_streams=4)
-    b = Ensemble(members, dt=dts, solver=SPEC, graph=True, max_streams=4)
+    b = Ensemble(members, dt=dts, solver=SPEC, graph=True, max_streams=4, lu_bs=4)
     for m in range(len(members)):
         a.set_state(m, W[m])
         b.set_state(m, W[m])
     tune = a.autotune(steps=1)
     print(f"autotune: {tune}")
-    assert len(tune["trial_ms"]) == 8 and tune["nstreams"] in (1, 2, 3, 4)
-    assert tune["lu_bs"] in (4, 8)
+    # one trial a stream count; the unroll option selects nothing and is reported
+    assert len(tune["trial_ms"]) == 4 and tune["nstreams"] in (1, 2, 3, 4)
+    assert tune["trial_ms"][tune["nstreams"] - 1] == min(tune["trial_ms"])
+    assert tune["lu_bs"] == 8 and b.tuning()["lu_bs"] == 4
     a.step(2)
     b.step(2)
     for m in range(len(members)):
