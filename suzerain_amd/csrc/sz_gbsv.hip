@@ -463,25 +463,16 @@ void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
              const cpx<R> *__restrict__ ab, int ldab, long long sab,
              const int *__restrict__ ipiv, long long sipiv,
              cpx<R> *__restrict__ b, int ldb, long long sb,
-             const int *__restrict__ skip, int nsys,
-             const sz::gsys *__restrict__ gs = nullptr)
+             const int *__restrict__ skip, int nsys)
 {
     using T = cpx<R>;
     extern __shared__ __align__(16) unsigned char smem[];
     const int sys = blockIdx.x;
     if (sys >= nsys) return;
     if (skip && skip[sys] != 0) return;   // singular factor: leave b as is
-    if (gs) {                             // grouped: per-system order, storage
-        const sz::gsys g = gs[sys];
-        n = g.n;
-        ab = reinterpret_cast<const T *>(g.ab);
-        ipiv = reinterpret_cast<const int *>(g.ipiv);
-        b = reinterpret_cast<T *>(g.b);
-    } else {
-        ab += (size_t)sys * (size_t)sab;
-        ipiv += (size_t)sys * (size_t)sipiv;
-        b += (size_t)sys * (size_t)sb;
-    }
+    ab += (size_t)sys * (size_t)sab;
+    ipiv += (size_t)sys * (size_t)sipiv;
+    b += (size_t)sys * (size_t)sb;
     const int tid = threadIdx.x;
     const int kv = kl + ku;
     T *x = reinterpret_cast<T *>(smem);
@@ -631,7 +622,8 @@ void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
 //   * SOLVE_LT: the L^T half alone, after a factorization that solved U^T.
 // The columns of the next PF steps are in flight: the barrier to the scheduler
 // before each fetch keeps a load behind the last use of the registers it fills
-// (else they are copied, and the copy waits for the load).
+// (else they are copied, and the copy waits for the load), and the first PF
+// fetches in their order (else the first step of every PF waits for all).
 // Bound by instruction issue of one wavefront (75 instructions a step; the
 // division by U(j, j) has its reciprocal formed 64 at a time), for thousands of
 // systems by issue of the SIMD; the factors' bytes take a third of the time.
@@ -784,7 +776,7 @@ __global__ __launch_bounds__(64)
 void k_gbtrs_reg(int trans, int n, int kl, int ku, int nrhs, const cpx<R> *__restrict__ ab,
                  int ldab, long long sab, const int *__restrict__ ipiv, long long sipiv,
                  cpx<R> *__restrict__ b, int ldb, long long sb,
-                 const int *__restrict__ skip, int nsys, const sz::gsys *__restrict__ gs)
+                 const int *__restrict__ skip, int nsys)
 {
     using T = cpx<R>;
     constexpr int PF = 8;                    // columns requested ahead
@@ -793,17 +785,9 @@ void k_gbtrs_reg(int trans, int n, int kl, int ku, int nrhs, const cpx<R> *__res
     const int sys = blockIdx.x;
     if (sys >= nsys) return;
     if (skip && skip[sys] != 0) return;      // singular factor: leave b as is
-    if (gs) {                                // grouped: per-system order, storage
-        const sz::gsys g = gs[sys];
-        n = g.n;
-        ab = reinterpret_cast<const T *>(g.ab);
-        ipiv = reinterpret_cast<const int *>(g.ipiv);
-        b = reinterpret_cast<T *>(g.b);
-    } else {
-        ab += (size_t)sys * (size_t)sab;
-        ipiv += (size_t)sys * (size_t)sipiv;
-        b += (size_t)sys * (size_t)sb;
-    }
+    ab += (size_t)sys * (size_t)sab;
+    ipiv += (size_t)sys * (size_t)sipiv;
+    b += (size_t)sys * (size_t)sb;
     const int lane = threadIdx.x, kv = kl + ku;
     const bool cj = trans == 2;
     // xs[i], zero outside 0 .. n-1
@@ -846,6 +830,7 @@ void k_gbtrs_reg(int trans, int n, int kl, int ku, int nrhs, const cpx<R> *__res
                 };
                 unroll<PF>([&](auto u_) __attribute__((always_inline)) {
                     fetch(decltype(u_)::value, qx[decltype(u_)::value], qy[decltype(u_)::value]);
+                    __builtin_amdgcn_sched_barrier(0);
                 });
                 for (int j0 = 0; j0 < n; j0 += 64) {
                     for (int jj0 = 0; jj0 < 64 && j0 + jj0 < n; jj0 += PF) {
@@ -1051,6 +1036,7 @@ void k_gbtrs_reg(int trans, int n, int kl, int ku, int nrhs, const cpx<R> *__res
                 unroll<PF>([&](auto u_) __attribute__((always_inline)) {
                     constexpr int u = decltype(u_)::value;
                     fetch(n - 2 - u, qx[u], qy[u]);
+                    __builtin_amdgcn_sched_barrier(0);
                 });
                 int j = n - 2;
                 for (int jt = n - 2; jt >= 0; jt -= 64) {
@@ -2288,24 +2274,25 @@ bool launch_gbtrs_t16(int tc, int n, int kl, int ku, const void *ab, int ldab,
 
 // The register solve where the band fits its lanes, else false (k_gbtrs takes
 // any band its staging holds; it is the slower at every band both take, see
-// k_gbtrs_reg).  nmax: the longest right hand side (its LDS).
+// k_gbtrs_reg).
 template <typename R>
 bool launch_gbtrs_reg(int tc, int n, int kl, int ku, int nrhs, const void *ab, int ldab,
                       long long sab, const int *ipiv, long long sipiv, void *b, int ldb,
-                      long long sb, const int *skip, int nsys, int nmax,
-                      const sz::gsys *gs, hipStream_t stream, bool lt_only = false)
+                      long long sb, const int *skip, int nsys, hipStream_t stream,
+                      bool lt_only = false)
 {
     const int kv = kl + ku;
     // the transposed ones keep finished rows to the end of a block of four (U^T)
     // and of eight (L^T)
     if (tc == 0 ? kl > 63 || kv > 127 : kl > 56 || kv > 124) return false;
-    const size_t lds = (size_t)nmax * sizeof(cpx<R>);
+    const size_t lds = (size_t)n * sizeof(cpx<R>);
 #define SZ_REG(MODE_, NR_)                                                        \
     hipLaunchKernelGGL((k_gbtrs_reg<R, MODE_, NR_>), dim3(nsys), dim3(64), lds, stream, tc, \
                        n, kl, ku, nrhs, reinterpret_cast<const cpx<R> *>(ab), ldab, sab, \
-                       ipiv, sipiv, reinterpret_cast<cpx<R> *>(b), ldb, sb, skip, nsys, gs)
-    if (lt_only) {
-        SZ_REG(SOLVE_LT, 1);
+                       ipiv, sipiv, reinterpret_cast<cpx<R> *>(b), ldb, sb, skip, nsys)
+    if (lt_only) {                           // (the fused factorization is double)
+        if constexpr (sizeof(R) == 8) SZ_REG(SOLVE_LT, 1);
+        else return false;
     } else if (tc == 0) {
         if (kv <= 63) SZ_REG(SOLVE_N, 1);
         else SZ_REG(SOLVE_N, 2);
@@ -2348,7 +2335,7 @@ int launch_gbtrs(char trans, int n, int kl, int ku, int nrhs, const void *ab,
                             nsys, n, nullptr, stream))
         return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
     if (launch_gbtrs_reg<R>(tc, n, kl, ku, nrhs, ab, ldab, sab, ipiv, sipiv, b, ldb, sb,
-                            skip, nsys, n, nullptr, stream, lt_only))
+                            skip, nsys, stream, lt_only))
         return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
     if (lt_only) return SZ_ERR_LDS;          // only after a fused factorization
     if (tc == 0)
@@ -2366,8 +2353,9 @@ int launch_gbtrs(char trans, int n, int kl, int ku, int nrhs, const void *ab,
 
 // Grouped launches: every system of gs (orders up to nmax, band storage at
 // gs[s].ab with leading dimension ldab = 2 kl + ku + 1) in one launch.
-// The panel kernel takes the channel band shapes; no other is grouped.
-template <typename R>
+// The precision solver's float factors, the only ones it groups: the panel
+// kernel and the sixteen-lane solve take its band shapes at every order its
+// sweep takes.
 int launch_gbtrf_grouped(int kl, int ku, void *ab, int ldab, int *ipiv, int *info,
                          const int *skip, const sz::gsys *gs, int nsys,
                          hipStream_t stream)
@@ -2375,8 +2363,8 @@ int launch_gbtrf_grouped(int kl, int ku, void *ab, int ldab, int *ipiv, int *inf
     if (nsys <= 0) return nsys < 0 ? -10 : 0;
     if (ldab != 2 * kl + ku + 1) return -5;
     if (!((kl == 34 && ku == 34) || (kl == 24 && ku == 24))) return SZ_ERR_LDS;
-    if (!launch_panel<R, false>(0, kl, ku, ab, ldab, 0, ipiv, 0, info, skip, nsys, nullptr,
-                                0, gs, stream))
+    if (!launch_panel<float, false>(0, kl, ku, ab, ldab, 0, ipiv, 0, info, skip, nsys,
+                                    nullptr, 0, gs, stream))
         return SZ_ERR_LDS;
     return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
 }
@@ -2428,7 +2416,6 @@ void k_band_split(int kl, int ku, const sz::gsys *__restrict__ gs, int s0, int n
     }
 }
 
-template <typename R>
 int launch_gbtrs_grouped(char trans, int kl, int ku, const void *ab, int ldab,
                          const int *ipiv, void *b, const int *skip,
                          const sz::gsys *gs, int nsys, int nmax,
@@ -2437,19 +2424,9 @@ int launch_gbtrs_grouped(char trans, int kl, int ku, const void *ab, int ldab,
     const int tc = trans_code(trans);
     if (tc <= 0) return -1;              // the transposed solves only
     if (nsys <= 0) return nsys < 0 ? -10 : 0;
-    if (kl + ku + 1 > TRS_PRE * TRS_NT) return SZ_ERR_LDS;
-    const size_t lds = (size_t)nmax * sizeof(cpx<R>);
-    if (lds > LDS_MAX) return SZ_ERR_LDS;
-    if (launch_gbtrs_t16<R>(tc, 0, kl, ku, ab, ldab, 0LL, ipiv, 0LL, b, 0LL, skip, nsys,
-                            nmax, gs, stream))
-        return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
-    if (launch_gbtrs_reg<R>(tc, 0, kl, ku, 1, ab, ldab, 0LL, ipiv, 0LL, b, nmax, 0LL, skip,
-                            nsys, nmax, gs, stream))
-        return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
-    hipLaunchKernelGGL((k_gbtrs<R, true>), dim3(nsys), dim3(TRS_NT), lds, stream, tc,
-                       nmax, kl, ku, 1, reinterpret_cast<const cpx<R> *>(ab), ldab,
-                       0LL, ipiv, 0LL, reinterpret_cast<cpx<R> *>(b), nmax, 0LL, skip,
-                       nsys, gs);
+    if (!launch_gbtrs_t16<float>(tc, 0, kl, ku, ab, ldab, 0LL, ipiv, 0LL, b, 0LL, skip,
+                                 nsys, nmax, gs, stream))
+        return SZ_ERR_LDS;
     return hipGetLastError() == hipSuccess ? 0 : SZ_ERR_LAUNCH;
 }
 
@@ -2461,12 +2438,10 @@ int sz_internal_gbtrf_grouped(int single, int kl, int ku, void *ab, int ldab,
                               int *ipiv, int *info, const int *skip,
                               const void *gs, int nsys, void *stream)
 {
-    const sz::gsys *g = static_cast<const sz::gsys *>(gs);
-    if (single)
-        return launch_gbtrf_grouped<float>(kl, ku, ab, ldab, ipiv, info, skip, g,
-                                           nsys, (hipStream_t)stream);
-    return launch_gbtrf_grouped<double>(kl, ku, ab, ldab, ipiv, info, skip, g, nsys,
-                                        (hipStream_t)stream);
+    if (!single) return SZ_ERR_LDS;
+    return launch_gbtrf_grouped(kl, ku, ab, ldab, ipiv, info, skip,
+                                static_cast<const sz::gsys *>(gs), nsys,
+                                (hipStream_t)stream);
 }
 
 // 1 when the single precision grouped transposed solve of this band shape
@@ -2498,12 +2473,10 @@ int sz_internal_gbtrs_grouped(int single, char trans, int kl, int ku,
                               const int *skip, const void *gs, int nsys, int nmax,
                               void *stream)
 {
-    const sz::gsys *g = static_cast<const sz::gsys *>(gs);
-    if (single)
-        return launch_gbtrs_grouped<float>(trans, kl, ku, ab, ldab, ipiv, b, skip, g,
-                                           nsys, nmax, (hipStream_t)stream);
-    return launch_gbtrs_grouped<double>(trans, kl, ku, ab, ldab, ipiv, b, skip, g,
-                                        nsys, nmax, (hipStream_t)stream);
+    if (!single) return SZ_ERR_LDS;
+    return launch_gbtrs_grouped(trans, kl, ku, ab, ldab, ipiv, b, skip,
+                                static_cast<const sz::gsys *>(gs), nsys, nmax,
+                                (hipStream_t)stream);
 }
 
 int sz_zgbtrf_batched(int n, int kl, int ku, void *ab, int ldab,
