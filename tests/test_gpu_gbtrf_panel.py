@@ -1,4 +1,5 @@
-"""The panel factorization (four columns at a time) of the channel band shapes
+"""The panel factorization (four columns at a time) of the channel band shapes, alone
+and with U^T y = b solved on the way,
 where it can go wrong: orders around its block of four columns, its 64-column
 window and its last rows; pivots far enough to reach the columns beyond the
 window; zero pivots; and infinities, whose updates must leave the columns no
@@ -46,10 +47,12 @@ def _check(gpu, ab, kl, ku, precision):
     return ipiv
 
 
+ORDERS = [1, 2, 3, 4, 5, 35, 37, 63, 64, 65, 68, 69, 70, 71, 72, 73, 76, 103, 135]
+
+
 @pytest.mark.parametrize("precision", ["z", "c"])
 @pytest.mark.parametrize("kl,ku", SHAPES)
-@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 35, 37, 63, 64, 65, 68, 69, 70, 71,
-                               72, 73, 76, 103, 135])
+@pytest.mark.parametrize("N", ORDERS)
 def test_orders_around_the_blocks(gpu, N, kl, ku, precision):
     rng = np.random.default_rng(1000 * kl + ku + N)
     _check(gpu, _bands(rng, 3, N, kl, ku, 0.0), kl, ku, precision)
@@ -90,6 +93,79 @@ def test_infinities_and_zero_columns(gpu, kl, ku):
     _check(gpu, ab, kl, ku, "z")
 
 
+def _fused_entries():
+    """The factorization with U^T y = b, and the L^T sweep that completes it."""
+    import ctypes as C
+    from suzerain_amd._lib import load
+    lib = load()
+    i32, i64, vp = C.c_int, C.c_longlong, C.c_void_p
+    ut, lt = lib.sz_internal_zgbtrf_ut, lib.sz_internal_zgbtrs_lt
+    ut.restype = lt.restype = i32
+    ut.argtypes = [i32, i32, i32, vp, i32, i64, vp, i64, vp, vp, i64, i32, vp]
+    lt.argtypes = [i32, i32, i32, vp, i32, i64, vp, i64, vp, i64, vp, i32, vp]
+    return ut, lt
+
+
+def _check_fused(gpu, rng, ab, kl, ku):
+    """Factors, pivots and info against ZGBTRF, and the solutions of the systems
+    without a zero pivot against ZGBTRS 'T'.  Right hand sides a stride apart
+    that leaves a gap, which stays as it is."""
+    import ctypes as C
+    import torch
+    ut, lt = _fused_entries()
+    nb, N, ldab = ab.shape
+    b = rng.standard_normal((nb, N + 3)) + 1j * rng.standard_normal((nb, N + 3))
+    abd, bd = torch.from_numpy(ab).to(gpu), torch.from_numpy(b).to(gpu)
+    ipiv = torch.zeros((nb, N), dtype=torch.int32, device=gpu)
+    info = torch.full((nb,), -1, dtype=torch.int32, device=gpu)
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert ut(N, kl, ku, abd.data_ptr(), ldab, ldab * N, ipiv.data_ptr(), N,
+              info.data_ptr(), bd.data_ptr(), N + 3, nb, stream) == 0
+    assert lt(N, kl, ku, abd.data_ptr(), ldab, ldab * N, ipiv.data_ptr(), N,
+              bd.data_ptr(), N + 3, info.data_ptr(), nb, stream) == 0
+    lu, piv, x = abd.cpu().numpy(), ipiv.cpu().numpy(), bd.cpu().numpy()
+    info = info.cpu().numpy()
+    np.testing.assert_array_equal(x[:, N:], b[:, N:])
+    for s in range(nb):
+        ref = ab[s].reshape(-1).copy()
+        rinfo, rpiv = oracle.zgbtrf(N, kl, ku, ref, ldab)
+        assert info[s] == rinfo
+        np.testing.assert_array_equal(piv[s], rpiv)
+        np.testing.assert_array_equal(lu[s], ref.reshape(N, ldab))
+        if rinfo == 0:
+            want = oracle.zgbtrs("T", N, kl, ku, ref, ldab, rpiv, b[s, :N].copy())
+            np.testing.assert_array_equal(x[s, :N], want, err_msg=str((N, s)))
+    return piv, info
+
+
+@pytest.mark.parametrize("kl,ku", SHAPES)
+@pytest.mark.parametrize("N", ORDERS)
+def test_fused_orders_around_the_blocks(gpu, N, kl, ku):
+    """As test_orders_around_the_blocks, with U^T y = b on the way: a partial
+    last block's y, and the right hand sides handed over from the columns beyond
+    the window."""
+    rng = np.random.default_rng(2000 * kl + ku + N)
+    _check_fused(gpu, rng, _bands(rng, 3, N, kl, ku, 0.0), kl, ku)
+    _check_fused(gpu, rng, _bands(rng, 2, N, kl, ku, 20.0), kl, ku)
+
+
+@pytest.mark.parametrize("kl,ku", SHAPES)
+@pytest.mark.parametrize("N", [74, 150])
+def test_fused_far_pivots_and_singular_systems(gpu, N, kl, ku):
+    """Every pivot kl rows away; a zero column between two ordinary systems,
+    whose solutions it must not touch; a zero last column."""
+    rng = np.random.default_rng(3 * kl + ku + N)
+    ab = _bands(rng, 6, N, kl, ku, 0.0)
+    ab[0, :, 2 * kl + ku] *= 50.0
+    for j in range(N):                       # entries past the last row stay zero
+        ab[0, j, kl + ku + N - j:] = 0
+    ab[2, 30, :] = 0.0
+    ab[4, N - 1, :] = 0.0
+    piv, info = _check_fused(gpu, rng, ab, kl, ku)
+    assert (piv[0] - np.arange(1, N + 1)).max() == kl
+    assert [i > 0 for i in info] == [False, False, True, False, True, False]
+
+
 @pytest.mark.parametrize("kl,ku", SHAPES)
 def test_arrays_aligned_as_c_double_complex(gpu, kl, ku):
     """Band storage and right hand sides 8 bytes off a 16-byte boundary, which
@@ -99,11 +175,8 @@ def test_arrays_aligned_as_c_double_complex(gpu, kl, ku):
     import ctypes as C
     import torch
     from suzerain_amd._lib import load
-    lib = load()
-    i32, i64, vp = C.c_int, C.c_longlong, C.c_void_p
-    f_ut = lib.sz_internal_zgbtrf_ut
-    f_ut.restype = i32
-    f_ut.argtypes = [i32, i32, i32, vp, i32, i64, vp, i64, vp, vp, i64, i32, vp]
+    lib, vp = load(), C.c_void_p
+    f_ut, _ = _fused_entries()
     rng = np.random.default_rng(kl + 2 * ku)
     N, nb, ldab = 77, 2, 2 * kl + ku + 1
     ab = _bands(rng, nb, N, kl, ku, 0.0)
