@@ -411,11 +411,16 @@ __device__ __forceinline__ void lt_sweep(int n, int kl, int kv,
         };
         T l1[QP], l2[QP];
         int qp[QP];
+        // a zero the compiler takes for a lane's own: scalar loads would join
+        // the counter that every wait for LDS drains
+        int z = 0;
+        asm volatile("" : "+v"(z));
 #pragma unroll
         for (int u = 0; u < QP; ++u) {
             l1[u] = ab[laddr(n - 2 - u, tid)];
             l2[u] = ab[laddr(n - 2 - u, tid + TRS_NT)];
-            qp[u] = ipiv[max(n - 2 - u, 0)];
+            qp[u] = ipiv[max(n - 2 - u, 0) + z];
+            __builtin_amdgcn_sched_barrier(0);   // in order of use
         }
         for (int jb = n - 2; jb >= 0; jb -= QP) {
 #pragma unroll
@@ -447,7 +452,7 @@ __device__ __forceinline__ void lt_sweep(int n, int kl, int kv,
                 }
                 l1[u] = ab[laddr(j - QP, tid)];
                 l2[u] = ab[laddr(j - QP, tid + TRS_NT)];
-                qp[u] = ipiv[max(j - QP, 0)];
+                qp[u] = ipiv[max(j - QP, 0) + z];
                 LDS_BARRIER();
             }
         }
@@ -556,11 +561,14 @@ void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
                     return ok ? (size_t)(jj + t) * ldab + kv - t : 0;
                 };
                 T q1[QP], q2[QP], qd[QP];
+                int z = 0;                             // (as in lt_sweep)
+                asm volatile("" : "+v"(z));
 #pragma unroll
                 for (int u = 0; u < QP; ++u) {
                     q1[u] = ab[uaddr(u, t1)];
                     q2[u] = ab[uaddr(u, t2)];
-                    qd[u] = ab[(size_t)min(u, n - 1) * ldab + kv];
+                    qd[u] = ab[(size_t)min(u, n - 1) * ldab + kv + z];
+                    __builtin_amdgcn_sched_barrier(0);   // in order of use
                 }
                 T xn = x[0];
                 for (int jb = 0; jb < n; jb += QP) {
@@ -584,7 +592,7 @@ void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
                             x[j + t] = sz::cfnms(x[j + t], cj_if(ab[uaddr(j, t)], cj), y);
                         q1[u] = ab[uaddr(j + QP, t1)];
                         q2[u] = ab[uaddr(j + QP, t2)];
-                        qd[u] = ab[(size_t)min(j + QP, n - 1) * ldab + kv];
+                        qd[u] = ab[(size_t)min(j + QP, n - 1) * ldab + kv + z];
                         LDS_BARRIER();
                         if (kv == 0 && tid == 0 && j + 1 < n) xn = x[j + 1];
                     }
