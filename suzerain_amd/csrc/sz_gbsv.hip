@@ -2280,9 +2280,19 @@ bool launch_gbtrs_t16(int tc, int n, int kl, int ku, const void *ab, int ldab,
     }
 }
 
-// The register solve where the band fits its lanes, else false (k_gbtrs takes
-// any band its staging holds; it is the slower at every band both take, see
-// k_gbtrs_reg).
+// The register solve where the band fits its lanes and the order is worth its
+// fixed work (whole groups of 8 or 16 steps, two rounds of prefetches), else
+// false: k_gbtrs takes any band its staging holds.  Measured as register / LDS
+// time, both precisions, bands of 0 to 116 off-diagonals, one and three right
+// hand sides, mean / worst:
+//   N: order 1 1.0 to 2.0 / 2.5, order 2 0.9 to 1.1 / 1.3, order 3 0.8 to 1.0 /
+//     1.1, order 8 0.55 to 0.75 / 1.0;
+//   T, 600 systems: order 3 1.3 / 1.9, 5 1.05 / 1.3, 6 0.95 / 1.06, 8 0.8 / 1.0;
+//   T, 2,400 to 20,000 systems: order 3 1.9 / 2.8, 6 1.3 / 1.6, 9 1.05 / 1.2,
+//     11 1.05 / 1.3, 12 1.0 / 1.1, 16 0.75 / 0.9;
+//   T without an L half (kl = 0): 600 systems: order 6 1.0 / 1.4, 9 1.0 / 1.1;
+//     more: 12 1.1 / 1.3, 17 1.2 / 1.6, 24 0.95 / 1.2, 28 0.85 / 1.05, 33 1.0 / 1.2,
+//     40 0.85 / 1.05.
 template <typename R>
 bool launch_gbtrs_reg(int tc, int n, int kl, int ku, int nrhs, const void *ab, int ldab,
                       long long sab, const int *ipiv, long long sipiv, void *b, int ldb,
@@ -2293,6 +2303,9 @@ bool launch_gbtrs_reg(int tc, int n, int kl, int ku, int nrhs, const void *ab, i
     // the transposed ones keep finished rows to the end of a block of four (U^T)
     // and of eight (L^T)
     if (tc == 0 ? kl > 63 || kv > 127 : kl > 56 || kv > 124) return false;
+    const bool few = nsys <= 1024;           // at most one a SIMD: latency counts
+    const int from = tc == 0 ? 3 : kl > 0 ? (few ? 6 : 12) : (few ? 9 : 24);
+    if (n < from && !lt_only) return false;
     const size_t lds = (size_t)n * sizeof(cpx<R>);
 #define SZ_REG(MODE_, NR_)                                                        \
     hipLaunchKernelGGL((k_gbtrs_reg<R, MODE_, NR_>), dim3(nsys), dim3(64), lds, stream, tc, \

@@ -3,7 +3,7 @@ around the 64-row window, the block of four rows and the eight columns
 requested ahead; bands at the edges of one and two registers a lane; far
 pivots, zeros in the right hand side (whose columns are left out), singular
 systems left as they are.  Compared with the oracle bit for bit; the widest
-bands take the LDS kernel.
+bands, and the smallest orders, take the LDS kernel.
 """
 import numpy as np
 import pytest
@@ -56,6 +56,36 @@ def test_solves_at_the_window_edges(gpu, kl, ku, precision):
                     want = oracle.zgbtrs(trans, N, kl, ku, lu[s].reshape(-1).copy(), ldab,
                                          piv[s], b[s, r].copy())
                     np.testing.assert_array_equal(got[s, r], want, err_msg=str((trans, N, s, r)))
+
+
+@pytest.mark.parametrize("precision", ["z", "c"])
+@pytest.mark.parametrize("kl,ku", [(0, 0), (0, 70), (4, 4), (40, 30)])
+def test_smallest_orders_in_small_and_large_batches(gpu, kl, ku, precision):
+    """The smallest orders take the LDS kernel, up to a larger order for more
+    than 1,024 systems: a large batch and its parts give the same bits, and the
+    oracle's, on either side of each line."""
+    import torch
+    import suzerain_amd as sa
+    rng = np.random.default_rng(7 * kl + ku)
+    nb, nrhs, ldab = 1025, 2, 2 * kl + ku + 1
+    for N in (1, 2, 3, 5, 6, 8, 9, 11, 12, 23, 24):
+        lu, piv = _factored(rng, nb, N, kl, ku, precision)
+        b = (rng.standard_normal((nb, nrhs, N)) +
+             1j * rng.standard_normal((nb, nrhs, N))).astype(lu.dtype)
+        lud, pd = torch.from_numpy(lu).to(gpu), torch.from_numpy(piv).to(gpu)
+        for trans in "NTC":
+            bd = torch.from_numpy(b).to(gpu)
+            parts = bd.clone()
+            sa.gbtrs(trans, lud, kl, ku, pd, bd, precision=precision)
+            for i in (slice(0, 1024), slice(1024, nb)):
+                sa.gbtrs(trans, lud[i], kl, ku, pd[i], parts[i], precision=precision)
+            got = bd.cpu().numpy()
+            np.testing.assert_array_equal(parts.cpu().numpy(), got, err_msg=str((trans, N)))
+            for s in (0, nb - 1):
+                for r in range(nrhs):
+                    want = oracle.zgbtrs(trans, N, kl, ku, lu[s].reshape(-1).copy(), ldab,
+                                         piv[s], b[s, r].copy())
+                    np.testing.assert_array_equal(got[s, r], want, err_msg=str((trans, N, s)))
 
 
 @pytest.mark.parametrize("trans", ["N", "T"])
