@@ -40,8 +40,9 @@ namespace {
 using sz::zd;
 constexpr int NT = 256;
 constexpr int MAXF = 16;
-// LDS per block a plan may ask for: 80 KB admits the in-place 16-line z
-// tile at length 288 (78 KB, two blocks per CU)
+// LDS per block of the run-time-size kernels: two blocks per CU.  Their tiles
+// (two buffers and the twiddles) are halved until they fit: 16 z lines up to
+// length 155, 8 up to 301.
 constexpr size_t FFT_LDS = 80 * 1024;
 
 struct radix_plan {
@@ -416,8 +417,9 @@ __device__ __forceinline__ void dft(double (&x)[L], double (&y)[L])
         });
 }
 
-// Lines (pairs of lines in x) a block transforms: 128-byte runs and at most
-// 40 KB of LDS for the longest, so that four blocks fit a CU.
+// Lines (pairs of lines in x) a block transforms: runs of at least 128 bytes
+// and at most 40 KB of LDS up to length 288, so that four blocks fit a CU; 384
+// takes 48 to 51 KB, three blocks.
 constexpr int fft_lines(int n) { return n >= 160 ? 8 : n >= 48 ? 16 : 32; }
 constexpr int fft_threads(int n1, int n2)
 {
@@ -633,7 +635,15 @@ void k_fft_r2c2(fft_geom g, const zd *__restrict__ tw, const double *__restrict_
 }
 
 // The lengths run as two register passes and their factors: the 3/2 rule's
-// lengths of the grids in use (144 and 288 are those of 96^3 and 192^3).
+// lengths of grids of 8, 12, 16, 24, 32, 36, 48, 64, 72, 96, 108, 128, 144, 192
+// and 256 points, those of this repository's channels, ensembles and tests.  A
+// choice of what to instantiate, not what the method can take: any length of two
+// factors up to 24 could be added (32 = 8 4, 64 = 8 8, 128 = 16 8, 256 = 16 16,
+// 324 = 18 18, 432 = 24 18, 576 = 24 24).  Measured over both passes, 5 fields of
+// 4 million points, backward and forward: these from 24 up at 4.0 to 5.8 and 3.8
+// to 6.2 TB/s, but 162 at 2.7 and 3.4 and 384 at 3.5 and 3.6; the run-time-size
+// kernels at 1.6 to 2.2 and 1.9 to 2.7 (32 to 256) and 0.9 to 1.4 and 1.1 to 1.6
+// TB/s (324 to 768), the rate they had before.
 #define SZ_FFT_TWO_PASS(X)                                                      \
     X(12, 4, 3) X(18, 6, 3) X(24, 6, 4) X(36, 6, 6) X(48, 8, 6) X(54, 9, 6)      \
     X(72, 9, 8) X(96, 12, 8) X(108, 12, 9) X(144, 16, 9) X(162, 18, 9)           \
@@ -714,8 +724,8 @@ sz_fft_plan *sz_fft_plan_create(int Ny, int Nx, int dNx, int Nz, int dNz,
     g.Xw = dNx / 2 + 1;
     g.xkeep = (Nx - 1) / 2 + 1;
     g.zabs = (Nz - 1) / 2;
-    // z: 16 lines per block (256-byte runs of y), or 8 with
-    // SZ_FFT_ZLINES=8; x: 8 (measured faster for the c2r/r2c pair at 144)
+    // tiles of the run-time-size kernels (the two-pass ones have their own).
+    // z: 16 lines per block (256-byte runs of y), or 8 with SZ_FFT_ZLINES=8; x: 8
     int yt = 16;
     if (const char *e = std::getenv("SZ_FFT_ZLINES"))
         if (std::atoi(e) == 8) yt = 8;

@@ -42,17 +42,31 @@ def test_transforms_match_numpy(gpu, Ny, Nx, Nz):
 
 
 @pytest.mark.parametrize("Ny,Nx,Nz", [(96, 96, 96), (7, 192, 192)])
-def test_eight_line_z_tiles(gpu, monkeypatch, Ny, Nx, Nz):
-    # SZ_FFT_ZLINES=8 selects the 8-line z tile at plan creation
+def test_eight_lines_leave_two_pass_lengths(gpu, monkeypatch, Ny, Nx, Nz):
+    # SZ_FFT_ZLINES=8 is for the run-time-size kernels; 144 and 288 have none
     monkeypatch.setenv("SZ_FFT_ZLINES", "8")
     _check_transforms(gpu, Ny, Nx, Nz)
 
 
-def _check_transforms(gpu, Ny, Nx, Nz):
+@pytest.mark.parametrize("zlines", ["", "8"])
+@pytest.mark.parametrize("Ny,dNx,dNz", [(96, 64, 128), (7, 128, 64), (13, 32, 81),
+                                        (29, 256, 27), (16, 8, 9), (5, 324, 256),
+                                        (1, 16, 432)])
+def test_run_time_size_kernels(gpu, monkeypatch, Ny, dNx, dNz, zlines):
+    """Lengths without two register passes, in z tiles of 16 lines and, by
+    SZ_FFT_ZLINES=8 at plan creation (lengths up to 155; 256 and 432 take 8 and 4
+    lines of themselves), of 8; numbers of lines that leave a tile partly filled."""
+    from test_gpu_fft_two_pass import LENGTHS
+    assert dNx not in LENGTHS and dNz not in LENGTHS
+    monkeypatch.setenv("SZ_FFT_ZLINES", zlines)
+    _check_transforms(gpu, Ny, 2 * dNx // 3, 2 * dNz // 3, dNx, dNz)
+
+
+def _check_transforms(gpu, Ny, Nx, Nz, dNx=None, dNz=None):
     import torch
     from suzerain_amd.fft import PencilFFT
-    print(f"case Ny={Ny} Nx={Nx} Nz={Nz}", flush=True)
-    dNx, dNz = 3 * Nx // 2, 3 * Nz // 2
+    dNx, dNz = dNx or 3 * Nx // 2, dNz or 3 * Nz // 2
+    print(f"case Ny={Ny} Nx={Nx} dNx={dNx} Nz={Nz} dNz={dNz}", flush=True)
     rng = np.random.default_rng(Ny + Nx)
     nf = 3
     W, keep = dealiased_wave(rng, nf, Ny, Nx, dNx, Nz, dNz)
