@@ -173,7 +173,9 @@ def lu_kernel_name(KL, KU, fused_ut=False):
     sel = os.environ.get("SZ_GBTRF_KERNEL", "")
     if sel.startswith("l") or (KL, KU) not in ((34, 34), (24, 24), (34, 20)):
         return "k_gbtrf<double, 256>"
-    return f"k_gbtrf_panel<double, {KL + 1}, {KL + KU}, {str(fused_ut).lower()}>"
+    waves = 3 if KL == 24 and not fused_ut else 2         # per SIMD
+    return (f"k_gbtrf_panel<double, {KL + 1}, {KL + KU}, "
+            f"{str(fused_ut).lower()}, {waves}>")
 
 
 # HBM bytes per LU launch measured with FETCH_SIZE/WRITE_SIZE PMC passes and

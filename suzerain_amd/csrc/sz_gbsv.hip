@@ -639,6 +639,9 @@ void k_gbtrs(int trans, int n, int kl, int ku, int nrhs,
 // kl = ku = 34: 459 -> 294 us (455 MB); T of 600 systems n = 301, kl 17, ku 11,
 // two right hand sides: 615 -> 253 us; L^T of 4560 systems n = 480, kl = 34:
 // 483 -> 334 us; N in float, 300 systems n = 200, kl = ku = 24: 37 -> 19 us.
+// What it loses: an element that is zero still costs N a step, where k_gbtrs left
+// its column out (an all-zero right hand side, kl = 0, 1500 systems n = 480: 53
+// -> 186 us).
 template <typename R>
 __device__ __forceinline__ R sel(bool c, R a, R b) { return c ? a : b; }
 
@@ -1413,21 +1416,26 @@ void k_gbtrs_t16(int n, const cpx<R> *__restrict__ ab, int ldab, long long sab,
 //      fused multiply-add itself: no readlane and no LDS read per multiplier
 //      (two readlanes cost as much as a multiply-add: 13.8 against 6.0 cycles
 //      for the pair, measured).
-//   3. U rows leave and the next rows enter as 64 contiguous bytes per column
-//      (one element at a time moved 2.5 times the bytes: 15.9 GB per 4560
-//      systems against 6.3 now and 6.1 needed), the rows straight to LDS
-//      early in the block so that no wait for them falls on the stores; the
-//      slots are renamed by four.
+//   3. U rows leave and the next rows enter as 64 contiguous bytes per column,
+//      the rows straight to LDS early in the block so that no wait for them
+//      falls on the stores; the slots are renamed by four.  (One element at a
+//      time moved 15.9 GB per 4560 systems fused, now 9.4 of 6.1 needed.  The
+//      writes are what is needed, 3.8; 5.7 are read for 2.5: a miss brings a
+//      128-byte line, whose other half is asked for four columns later, when it
+//      has mostly left the L2.)
 // Every updated element sees the fnms sequence of the unblocked loop.
 //
-// What bounds it: vector issue, about 300 instructions per column step, 136
-// of them the multiply-adds of step 2 (they alone would take a fifth of the
-// time).  At two waves per SIMD (the window takes 152 of a lane's registers)
-// the pivot chain of one wave runs beside the updates of the other.  4560
-// systems of N = 480, kl = ku = 34, diagonally dominant: 2.85 ms, fused with
-// U^T 3.07 ms (an unblocked loop with readlane multipliers: 5.15 and 5.40
-// ms); 1152 systems 1.01 (1.50), one system 0.76 with U^T (1.21); complex
-// float 2.49 (5.37).
+// What bounds it: instruction issue and the pivot chain.  A column step of the
+// fused kernel on the channel's operator is 440 vector instructions, 103 scalar
+// and 35 of LDS (counters); 136 of them are the multiply-adds of step 2, which
+// alone would take a quarter of the time: 13.4 TF/s of the 72.6 a large product
+// reaches.  At two waves per SIMD (the window takes 152 of a lane's registers)
+// the pivot chain of one wave runs beside the updates of the other and the
+// vector unit is busy 70% of the time; of 4560 systems 464 are left for a third
+// round of single waves.  N = 480, kl = ku = 34, diagonally dominant, alone and
+// fused with U^T: 4560 systems 2.84 and 3.07 ms (an unblocked loop with readlane
+// multipliers: 5.15 and 5.40), 2048 1.16 and 1.24, 1152 0.97 (1.50) and 1.10,
+// one 0.66 and 0.75 (1.21); complex float 2.47 for 4560 (5.37).
 //
 // UT = true also solves U^T y = b on the way (the first half of ZGBTRS 'T'):
 // lane l keeps the pending b of its column, y_j = b_j / U(j,j) is formed with

@@ -719,11 +719,12 @@ void k_imexop_pack_listed(const gmember *__restrict__ mem, int nm,
 // block's systems.  Two blocks of AP_NT stay on a CU where their LDS fits, so
 // one loads while the other computes; else one of AP_NT1 (see apply_blocks).
 // Bound by latency at three waves a SIMD (the 1,150 instructions of a row are
-// a third of the time, the bytes a third to a half).  Measured, against one
-// system a block of 1,024 threads with weights formed from tables in LDS: 4,560
-// systems n = 96 130 -> 77 us (0.36 GB), 18,336 systems n = 192 1080 -> 485 us
-// and their refinement sweep 840 -> 406 us; of which 840 -> 490 by the constant
-// structure, the rest by y and b requested before the products.
+// a third of the time, the bytes another).  Measured, against one system a block
+// of 1,024 threads with weights formed from tables in LDS: 4,560 systems n = 96
+// 130 -> 69 us (x, y and the result 0.105 GB; 77 us as a channel calls it, with
+// the pencils' offsets), 18,336 systems n = 192 1080 -> 485 us and their
+// refinement sweep 840 -> 406 us; of which 840 -> 490 by the constant structure,
+// the rest by y and b requested before the products.
 constexpr int AP_NT = 384, AP_NT1 = 768;
 #define AP_BOUNDS(NT_) __launch_bounds__(NT_) __attribute__((amdgpu_waves_per_eu(3, 3)))
 

@@ -659,7 +659,12 @@ void rebuild(sz_prec *h)
         (void)hipMemcpy(h->D, D.data(), D.size() * sizeof(pdesc),
                         hipMemcpyHostToDevice);
     // the single precision solve reads split factors where it can: a
-    // class's factors are converted after every factorization
+    // class's factors are converted after every factorization.  That pays
+    // where factors are kept: a solve of 4,560 systems N = 480 takes 0.406 ms
+    // instead of 0.464 and their conversion 2.6, the gain of 45 solves or some
+    // 18 steps.  Without reuse a factor serves siter + 1 solves at most, and the
+    // conversion is a loss (840 systems N = 365, k = 6: 206 us beside the 400 us
+    // of all four solves).
     long long stemp = 0;
     for (auto &c : h->classes) {
         c.split = sz_internal_gbtrs_split_ok(c.KL, c.KU, c.nmax);

@@ -61,10 +61,9 @@ def test_members_equal_alone(gpu, graph):
 
 
 def test_members_on_every_sweep_tier(gpu):
-    """The refinement sweep runs one launch per LDS tier of system sizes
-    (profiles staged with two blocks per CU, gathered with two, staged with
-    one): members on every tier, side by side, still equal their solo runs
-    bit for bit, replayed."""
+    """The refinement sweep runs one launch per tier of system sizes (two
+    blocks fit a CU; one block holds two systems; the rest): members on every
+    tier, side by side, still equal their solo runs bit for bit, replayed."""
     from suzerain_amd._lib import load
     from suzerain_amd.channel import DEFAULT_SCENARIO
     from suzerain_amd.ensemble import Ensemble, default_dt
