@@ -54,3 +54,43 @@ def test_apply_matches_oracle(gpu, n, k, nsys):
                                          np.ascontiguousarray(x[:, s]), beta, want,
                                          present=present)
             np.testing.assert_array_equal(got[:, s], want, err_msg=str((s, beta, present)))
+
+
+@pytest.mark.parametrize("n", [24, 96, 260])
+def test_strided_profiles_and_scattered_pencils(gpu, n):
+    """Profiles a stride apart and pencils at offsets of their own, input and
+    output at different ones, in place where they are the same: the same bits as
+    the contiguous call, and nothing else written."""
+    import torch
+    import suzerain_amd as sa
+    from suzerain_amd.imexop import Imexop
+    rng = np.random.default_rng(n)
+    nsys, beta = 37, 0.5 - 2j
+    imx = Imexop(sa.BsplineOp.channel(n, 8, 3.0), *SCEN)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    crand = lambda *s: rng.standard_normal(s) + 1j * rng.standard_normal(s)
+    refs = rng.uniform(-1, 1, (26, n))
+    km, kn = dev(rng.uniform(-30, 30, nsys)), dev(rng.uniform(-30, 30, nsys))
+    x, y = crand(5, nsys, n), crand(5, nsys, n)
+    want = dev(y)
+    imx.accumulate(PHI, km, kn, dev(refs), dev(x), beta, want)
+    want = want.cpu().numpy()
+    strided = dev(refs.T).T                          # (26, n), stride(1) = 26
+    assert strided.stride(1) == 26
+    place = lambda: rng.permutation(2 * nsys)[:nsys] * (n + 3)
+    io, oo = place(), place()
+    xb, yb = crand(5, 2 * nsys * (n + 3)), crand(5, 2 * nsys * (n + 3))
+    for s in range(nsys):
+        xb[:, io[s]:io[s] + n] = x[:, s]
+        yb[:, oo[s]:oo[s] + n] = y[:, s]
+    yd = dev(yb)
+    imx.accumulate(PHI, km, kn, strided, list(dev(xb)), beta, list(yd), nsys=nsys,
+                   inoff=dev(io), outoff=dev(oo))
+    for s in range(nsys):
+        yb[:, oo[s]:oo[s] + n] = want[:, s]
+    np.testing.assert_array_equal(yd.cpu().numpy(), yb)
+    xd = dev(x)                                      # y = (M + phi L) x + beta x
+    imx.accumulate(PHI, km, kn, dev(refs), xd, beta, xd)
+    other = dev(x)
+    imx.accumulate(PHI, km, kn, dev(refs), dev(x), beta, other)
+    np.testing.assert_array_equal(xd.cpu().numpy(), other.cpu().numpy())
