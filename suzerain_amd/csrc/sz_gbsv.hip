@@ -2293,11 +2293,11 @@ bool launch_gbtrs_t16(int tc, int n, int kl, int ku, const void *ab, int ldab,
 // false: k_gbtrs takes any band its staging holds.  Measured as register / LDS
 // time, both precisions, bands of 0 to 116 off-diagonals, one and three right
 // hand sides, mean / worst:
-//   N: order 1 1.0 to 2.0 / 2.5, order 2 0.9 to 1.1 / 1.3, order 3 0.8 to 1.0 /
-//     1.1, order 8 0.55 to 0.75 / 1.0;
+//   N: order 1 1.0 to 2.0 / 2.5, order 2 0.9 to 1.2 / 1.5, order 3 0.8 to 1.1 /
+//     1.3, order 8 0.55 to 0.8 / 1.0;
 //   T, 600 systems: order 3 1.3 / 1.9, 5 1.05 / 1.3, 6 0.95 / 1.06, 8 0.8 / 1.0;
-//   T, 2,400 to 20,000 systems: order 3 1.9 / 2.8, 6 1.3 / 1.6, 9 1.05 / 1.2,
-//     11 1.05 / 1.3, 12 1.0 / 1.1, 16 0.75 / 0.9;
+//   T, 2,400 to 20,000 systems: order 3 1.6 to 2.4 / 2.8, 6 1.3 / 1.6, 9 1.05 /
+//     1.2, 11 1.05 / 1.3, 12 1.0 / 1.1, 16 0.75 / 0.9;
 //   T without an L half (kl = 0): 600 systems: order 6 1.0 / 1.4, 9 1.0 / 1.1;
 //     more: 12 1.1 / 1.3, 17 1.2 / 1.6, 24 0.95 / 1.2, 28 0.85 / 1.05, 33 1.0 / 1.2,
 //     40 0.85 / 1.05.
