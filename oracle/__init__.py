@@ -1,7 +1,7 @@
 """CPU oracle for the suzerain banded-implicit hot path.
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and
-bench.py's cpu_baseline leg as the checker or the timed CPU baseline.  The
+bench.py's cpu_baseline leg as the oracle or the timed CPU baseline.  The
 product package (suzerain_amd) never imports it.
 
 * ``liboracle.so`` (oracle.c): scalar C99 restatement of bsmbsm q/permute/

@@ -5,7 +5,7 @@
  * TEST INFRASTRUCTURE ONLY.  Nothing in the product (the suzerain_amd
  * package, its HIP kernels or its C ABI) links, loads or calls this file.
  * Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg use
- * it, as the checker or the timed CPU baseline.
+ * it, as the oracle or the timed CPU baseline.
  *
  * Restates, group of terms by group of terms:
  *   sz_or_imexop_accumulate   suzerain/rholut_imexop.c:43-531

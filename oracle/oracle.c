@@ -4,7 +4,7 @@
  * TEST INFRASTRUCTURE ONLY.  Nothing in the product (the suzerain_amd
  * package, its HIP kernels or its C ABI) links, loads or calls this file.
  * Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg use
- * it, and then only as the checker or as the timed CPU baseline.
+ * it, and then only as the oracle or as the timed CPU baseline.
  *
  * Plain scalar C99 restatement of the reference algorithms:
  *
